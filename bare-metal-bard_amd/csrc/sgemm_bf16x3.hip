@@ -28,13 +28,8 @@
 // [row][k] with k contiguous (row = m for A, n for B), so every fragment is
 // one 128-bit read. Rows are 64 bytes with their 16-byte chunks XOR-swizzled
 // by row (lds_off), so neither the fragment reads nor the staging stores
-// conflict on banks. A (k contiguous
-// in global memory) is staged with 128-bit loads, four k per lane, split and
-// written as two 64-bit stores. B (n contiguous) is staged as 4 x 4 blocks:
-// four 128-bit loads (rows k..k+3, columns n..n+3; a wave covers 32
-// consecutive column blocks of two k rows, so each load is two 512-byte
-// coalesced accesses), a transpose in registers, then per column one 64-bit
-// store of its 4 k per plane.
+// conflict on banks. How an operand gets there (OpStage) depends on whether
+// k or m/n is contiguous in memory.
 //
 // Schedule: double-buffered LDS stages with register prefetch; one barrier
 // per stage. While a stage is consumed, the next one is split and stored from
@@ -47,6 +42,17 @@
 // conversion ran after them, so the two waves of a SIMD, kept in phase by the
 // barrier, converted at the same time while the matrix core idled. The fenced
 // order is 1-5% faster on the GPT-2 shapes and 2% at N = 4096, bit-identical.
+//
+// What bounds it. With the device full of 128- or 256-wide tiles: power. On
+// N(0, 1) data at N = 4096 the matrix cores are busy 74% of the cycles while
+// the clock falls to 1.7 GHz (2.38 GHz on zeros, 24% faster at the same
+// cycles), so what counts is the energy of everything around the MFMAs.
+// Taking instructions out of the staging (split4 on pairs, loads without
+// address arithmetic, two stages per loop turn) gave 4-5% on 256 x 256 and
+// 6-9% on 128-wide tiles (per 32-k stage and CU: 2.50 -> 2.37 us, 1.42 ->
+// 1.33, 1.62 -> 1.48 for two 128 x 128). With few tiles: the latency chain of
+// a stage (0.4 us for a lone 64 x 64 workgroup against 0.09 of MFMAs), which
+// more resident workgroups overlap and a deeper prefetch does not shorten.
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -69,6 +75,8 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 using bmb::f32x16;
 
 constexpr int BK = 32;   // k per LDS stage: two 16-k MFMA steps
@@ -135,13 +143,25 @@ constexpr float BF16_FINITE_MAX = 0x1.fefffep+127f;
 // finite x still splits exactly instead of into (inf, -inf), and an infinite
 // x gives (+-3.39e38, +-inf), whose products with a nonzero b are +-inf and
 // with b = 0 NaN, as in fp32. NaN stays NaN in lo.
+//
+// Written on pairs: one v_cvt_pk_bf16_f32 rounds two values, and its result is
+// widened again with a shift and a mask (12 instructions per four values
+// beside the clamps; asked for one value at a time the compiler converted
+// every hi twice, 20 in all).
 __device__ __forceinline__ void split4(const float (&x)[4], bf16x4 &hi, bf16x4 &lo) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const __bf16 h =
-            (__bf16)__builtin_amdgcn_fmed3f(x[i], -BF16_FINITE_MAX, BF16_FINITE_MAX);
-        hi[i] = h;
-        lo[i] = (__bf16)(x[i] - (float)h);
+    for (int i = 0; i < 4; i += 2) {
+        const f32x2 c = {__builtin_amdgcn_fmed3f(x[i], -BF16_FINITE_MAX, BF16_FINITE_MAX),
+                         __builtin_amdgcn_fmed3f(x[i + 1], -BF16_FINITE_MAX, BF16_FINITE_MAX)};
+        const bf16x2 h = __builtin_convertvector(c, bf16x2);
+        const unsigned u = __builtin_bit_cast(unsigned, h);
+        const f32x2 r = {x[i] - __builtin_bit_cast(float, u << 16),
+                         x[i + 1] - __builtin_bit_cast(float, u & 0xffff0000u)};
+        const bf16x2 l = __builtin_convertvector(r, bf16x2);
+        hi[i] = h[0];
+        hi[i + 1] = h[1];
+        lo[i] = l[0];
+        lo[i + 1] = l[1];
     }
 }
 
@@ -154,22 +174,54 @@ __device__ __forceinline__ void static_for(F &&f) {
     }
 }
 
+// A buffer descriptor over an operand from p on (uniform). The staging loads
+// go through it because they then take a uniform base that the scalar unit
+// advances per stage and a loop-invariant 32-bit offset per lane; with plain
+// pointers every load cost two 64-bit vector adds per stage. The loads stay
+// inside the operand by their offsets, so the descriptor's size does not
+// bound them.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t operand(const float *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, 0xffffffff, 0x00027000);
+}
+
 // Staging of one operand's tile per stage: ROWS rows (m of A, n of B) x BK k,
 // into a hi and a lo plane. KCONT: k is the contiguous axis of the stored
 // operand (A not transposed, B transposed): 128-bit loads of four k, split,
 // one 64-bit store per plane. Otherwise rows are contiguous (A transposed, B
-// not): 4 x 4 blocks (four k rows of four consecutive m or n; a wave covers
-// 32 consecutive blocks of two k rows, so each load is two 512-byte coalesced
-// accesses), transposed in registers, one 64-bit store of four k per row and
-// plane.
-template <int ROWS, int NT, bool KCONT, bool VEC>
+// not): blocks of 4 k x W rows (a wave covers 32 consecutive blocks of two k
+// rows), transposed in registers, one 64-bit store of four k per row and
+// plane. W is 4, or 2 where a tile has fewer 4 x 4 blocks than the workgroup
+// has lanes (64 rows on 256 lanes; see also Bf16x3Gemm::PAIR).
+//
+// IN (interior): all ROWS rows lie inside the operand. An edge tile loads
+// from clamped rows instead of checking bounds: LDS rows past the operand's
+// last one then hold copies of other rows, which only reach outputs that are
+// not stored. (A block that straddles the last row is loaded from further
+// back and shifted into place when it is split.) So edge tiles run the same
+// branch-free loop as interior ones; only a last stage with fewer than BK k
+// (load_tail) fills with zeros. Every path loads whole vectors and selects
+// from them afterwards: where a branch joined vectors loaded at once with
+// vectors loaded element by element, the compiler (ROCm 7.2) reused registers
+// of the former that were still live. That needs at least W rows and k, and
+// byte offsets below 2^32; EW (bf16x3_narrow_k) loads every element by itself.
+template <int ROWS, int NT, bool KCONT, bool IN, bool EW = false>
 struct OpStage {
-    static constexpr int CH = ROWS * BK / 4 / NT;      // KCONT: chunks per lane
-    static constexpr int BLK = BK * ROWS / 16;         // otherwise: 4 x 4 blocks per stage
+    static constexpr int CH = ROWS * BK / 4 / NT;  // KCONT: chunks per lane
+    static constexpr int W = !KCONT && ROWS * BK / 16 < NT ? 2 : 4;
+    static constexpr int BLK = BK * ROWS / (4 * W);    // otherwise: blocks per stage
     static constexpr int PER_T = (BLK + NT - 1) / NT;  // blocks per lane
     static constexpr int NLD = KCONT ? CH : 4 * PER_T;
     static_assert(!KCONT || (ROWS * BK / 4) % NT == 0, "staging splits evenly over the lanes");
-    float4 v[NLD];
+    static_assert(KCONT || BLK % NT == 0 || BLK < NT, "blocks split evenly over the lanes");
+    struct Vec {
+        float f[W];
+    };
+    Vec v[NLD];
+    // Byte offsets of this lane's loads from the stage's first element (row
+    // row0(), k 0), and how many rows before its place each block is loaded:
+    // loop-invariant.
+    unsigned o[NLD];
+    int shift[KCONT || IN ? 1 : PER_T];
 
     __device__ static __forceinline__ bool skip(int j, int tid) {
         return !KCONT && BLK % NT != 0 && tid + j * NT >= BLK;
@@ -179,27 +231,24 @@ struct OpStage {
         r = e / (BK / 4);
         c = (e % (BK / 4)) * 4;
     }
-    // Block e: k rows 4kb..4kb+3, rows rb..rb+3. Neighbouring lanes take the
-    // two halves of a 16-byte k chunk (kb even, odd) of one row block.
-    __device__ static __forceinline__ void block(int e, int &kb, int &rb) {
-        const int m = (e >> 1) % (ROWS / 4);
-        kb = 2 * ((e >> 1) / (ROWS / 4)) + (e & 1);
-        rb = 4 * m;
+    // Block e: k rows 4kb..4kb+3, rows W*m..W*m+W-1. Neighbouring lanes take
+    // the two halves of a 16-byte k chunk (kb even, odd) of one row block.
+    __device__ static __forceinline__ void block(int e, int &kb, int &row) {
+        const int m = (e >> 1) % (ROWS / W);
+        kb = 2 * ((e >> 1) / (ROWS / W)) + (e & 1);
+        row = W * m;
     }
-    __device__ static __forceinline__ float4 ld_in(const float *p) {
-        if (VEC) return bmb::ld4(p);
-        float4 x;
-        __builtin_memcpy(&x, p, sizeof(x));
-        return x;
-    }
-    // Byte offsets of this lane's loads from the stage base (row 0, k 0 of the
-    // tile): loop-invariant and 32-bit.
-    __device__ static __forceinline__ void offsets(unsigned (&o)[NLD], int ld, int tid) {
-        if (KCONT) {
+    // The row that offsets count from: the tile's first, or 0 where a clamped
+    // block may start before the tile.
+    __device__ static __forceinline__ int row0(int r0) { return IN || KCONT ? r0 : 0; }
+    // R rows in all, ld: the stored row stride, r0: the tile's first row.
+    __device__ __forceinline__ void setup(int R, int ld, int r0, int tid) {
+        if constexpr (KCONT) {
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 int r, c;
                 chunk(tid + i * NT, r, c);
+                if (!IN) r = min(r, R - 1 - r0);
                 o[i] = 4u * ((unsigned)r * (unsigned)ld + (unsigned)c);
             }
         } else {
@@ -207,131 +256,156 @@ struct OpStage {
             for (int j = 0; j < PER_T; ++j) {
                 int kb, rb;
                 block(min(tid + j * NT, BLK - 1), kb, rb);
+                if (!IN) {
+                    shift[j] = rb - min(rb, R - r0 - W);
+                    rb -= shift[j];
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    o[4 * j + i] = 4u * ((unsigned)(4 * kb + i) * (unsigned)ld + (unsigned)rb);
+                    o[4 * j + i] = 4u * ((unsigned)(4 * kb + i) * (unsigned)ld +
+                                         (unsigned)(rb + r0 - row0(r0)));
             }
         }
     }
-    // Interior stage: base = the stage's (row 0, k 0) element.
-    __device__ __forceinline__ void load_interior(const float *base, const unsigned (&o)[NLD],
-                                                  int tid) {
+    __device__ static __forceinline__ Vec ldv(__amdgpu_buffer_rsrc_t p, unsigned off) {
+        Vec x;
+        if constexpr (W == 4) {
+            const auto t = __builtin_amdgcn_raw_buffer_load_b128(p, (int)off, 0, 0);
+            __builtin_memcpy(&x, &t, sizeof(x));
+        } else {
+            const auto t = __builtin_amdgcn_raw_buffer_load_b64(p, (int)off, 0, 0);
+            __builtin_memcpy(&x, &t, sizeof(x));
+        }
+        return x;
+    }
+    // Elements n, n + 1, ... of x in its first places (n < W; what follows the
+    // last element is unspecified).
+    __device__ static __forceinline__ Vec shifted(const Vec &x, int n) {
+        Vec y;
+#pragma unroll
+        for (int c = 0; c < W; ++c) {
+            y.f[c] = x.f[c];
+#pragma unroll
+            for (int q = c + 1; q < W; ++q) y.f[c] = n == q - c ? x.f[q] : y.f[c];
+        }
+        return y;
+    }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t p, int tid) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i)
+            if (!skip(i / 4, tid)) v[i] = ldv(p, o[i]);
+    }
+    // EW: every element (row, k) by itself; rows past the last of R repeat it,
+    // k from rem (> 0) on are zeros. p: the stage's (row 0 of the operand,
+    // k 0) element.
+    __device__ __forceinline__ void load_single(const float *p, int R, int ld, int r0, int rem,
+                                                int tid) {
+        const auto at = [&](int r, int c) {
+            const size_t row = min(r0 + r, R - 1), k = min(c, rem - 1);
+            const float x = p[KCONT ? row * ld + k : k * ld + row];
+            return c < rem ? x : 0.0f;
+        };
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            int r, c;
+            if (KCONT) {
+                chunk(tid + i * NT, r, c);
+            } else {
+                block(tid + i / 4 * NT, c, r);
+                c = 4 * c + i % 4;
+            }
+#pragma unroll
+            for (int e = 0; e < W; ++e) v[i].f[e] = KCONT ? at(r, c + e) : at(r + e, c);
+        }
+    }
+    // A stage of which only the first rem (0 < rem < BK) k exist; the others
+    // become zero. p: the descriptor of the stage's base (KCONT: of the four
+    // elements before it; a chunk with fewer than four k is loaded as the
+    // stage's last four and shifted).
+    __device__ __forceinline__ void load_tail(__amdgpu_buffer_rsrc_t p, int ld, int rem, int tid) {
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             if (skip(i / 4, tid)) continue;
-            v[i] = ld_in(reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + o[i]));
-        }
-    }
-    // Zero fill outside the operand: P is the K range's origin, R its rows
-    // (M or N), K the range's length, ld the stored row stride.
-    __device__ __forceinline__ void load_guarded(const float *P, int R, int K, int ld, int r0,
-                                                 int k0, int tid) {
-        if (KCONT) {
-#pragma unroll
-            for (int i = 0; i < NLD; ++i) {
+            if constexpr (KCONT) {
                 int r, c;
                 chunk(tid + i * NT, r, c);
-                v[i] = bmb::load_chunk<VEC>(P, R, K, ld, r0 + r, k0 + c);
-            }
-        } else {
+                const int n = c - min(c, rem - 4);
+                v[i] = shifted(ldv(p, o[i] + 16u - 4u * (unsigned)n), n);
 #pragma unroll
-            for (int j = 0; j < PER_T; ++j) {
-                if (skip(j, tid)) continue;
-                int kb, rb;
-                block(tid + j * NT, kb, rb);
+                for (int e = 0; e < 4; ++e) v[i].f[e] = c + e < rem ? v[i].f[e] : 0.0f;
+            } else {
+                int kb, row;
+                block(tid + i / 4 * NT, kb, row);
+                const int k = 4 * kb + i % 4;
+                v[i] = ldv(p, o[i] - 4u * (unsigned)(k - min(k, rem - 1)) * (unsigned)ld);
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    v[4 * j + i] = bmb::load_chunk<VEC>(P, K, R, ld, k0 + 4 * kb + i, r0 + rb);
-            }
-        }
-    }
-    __device__ __forceinline__ void store(__bf16 *hi, __bf16 *lo, int tid) const {
-        if (KCONT) {
-#pragma unroll
-            for (int i = 0; i < NLD; ++i) {
-                int r, c;
-                chunk(tid + i * NT, r, c);
-                const float x[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-                bf16x4 h, l;
-                split4(x, h, l);
-                *reinterpret_cast<bf16x4 *>(hi + lds_off(r, c)) = h;
-                *reinterpret_cast<bf16x4 *>(lo + lds_off(r, c)) = l;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < PER_T; ++j) {
-                if (skip(j, tid)) continue;
-                int kb, rb;
-                block(tid + j * NT, kb, rb);
-                const float4 *b = v + 4 * j;
-                const float cols[4][4] = {{b[0].x, b[1].x, b[2].x, b[3].x},
-                                          {b[0].y, b[1].y, b[2].y, b[3].y},
-                                          {b[0].z, b[1].z, b[2].z, b[3].z},
-                                          {b[0].w, b[1].w, b[2].w, b[3].w}};
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    bf16x4 h, l;
-                    split4(cols[c], h, l);
-                    *reinterpret_cast<bf16x4 *>(hi + lds_off(rb + c, 4 * kb)) = h;
-                    *reinterpret_cast<bf16x4 *>(lo + lds_off(rb + c, 4 * kb)) = l;
-                }
+                for (int c = 0; c < W; ++c) v[i].f[c] = k < rem ? v[i].f[c] : 0.0f;
             }
         }
     }
-    // The store in pieces: chunk P (KCONT), or column P % 4 of block P / 4.
-    static constexpr int NPIECE = KCONT ? NLD : 4 * PER_T;
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) v[i] = Vec{};
+    }
+    // The split and its LDS stores in pieces: chunk P (KCONT), or row P % W of
+    // block P / W.
+    static constexpr int NPIECE = KCONT ? NLD : W * PER_T;
     template <int P>
     __device__ __forceinline__ void store_piece(__bf16 *hi, __bf16 *lo, int tid) const {
+        bf16x4 h, l;
         if constexpr (KCONT) {
             int r, c;
             chunk(tid + P * NT, r, c);
-            const float x[4] = {v[P].x, v[P].y, v[P].z, v[P].w};
-            bf16x4 h, l;
-            split4(x, h, l);
+            split4(v[P].f, h, l);
             *reinterpret_cast<bf16x4 *>(hi + lds_off(r, c)) = h;
             *reinterpret_cast<bf16x4 *>(lo + lds_off(r, c)) = l;
         } else {
-            constexpr int j = P / 4, c = P % 4;
+            constexpr int j = P / W, c = P % W;
             if (skip(j, tid)) return;
-            int kb, rb;
-            block(tid + j * NT, kb, rb);
-            const float4 *b = v + 4 * j;
-            auto col = [](const float4 &x) {
-                return c == 0 ? x.x : c == 1 ? x.y : c == 2 ? x.z : x.w;
-            };
-            const float x[4] = {col(b[0]), col(b[1]), col(b[2]), col(b[3])};
-            bf16x4 h, l;
+            int kb, row;
+            block(tid + j * NT, kb, row);
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                x[i] = IN || EW ? v[4 * j + i].f[c] : shifted(v[4 * j + i], shift[j]).f[c];
             split4(x, h, l);
-            *reinterpret_cast<bf16x4 *>(hi + lds_off(rb + c, 4 * kb)) = h;
-            *reinterpret_cast<bf16x4 *>(lo + lds_off(rb + c, 4 * kb)) = l;
+            *reinterpret_cast<bf16x4 *>(hi + lds_off(row + c, 4 * kb)) = h;
+            *reinterpret_cast<bf16x4 *>(lo + lds_off(row + c, 4 * kb)) = l;
         }
     }
-    // The interior loads into the registers that piece P was the last to read.
+    __device__ __forceinline__ void store(__bf16 *hi, __bf16 *lo, int tid) const {
+        static_for<0, NPIECE>([&](auto pc) { store_piece<decltype(pc)::value>(hi, lo, tid); });
+    }
+    // The loads into the registers that piece P was the last to read.
     template <int P>
-    __device__ __forceinline__ void load_after_piece(const float *base, const unsigned (&o)[NLD],
-                                                     int tid) {
-        auto at = [&](int i) {
-            return reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + o[i]);
-        };
+    __device__ __forceinline__ void load_after_piece(__amdgpu_buffer_rsrc_t p, int tid) {
         if constexpr (KCONT) {
-            v[P] = ld_in(at(P));
-        } else if constexpr (P % 4 == 3) {
-            constexpr int j = P / 4;
+            v[P] = ldv(p, o[P]);
+        } else if constexpr (P % W == W - 1) {
+            constexpr int j = P / W;
             if (skip(j, tid)) return;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[4 * j + i] = ld_in(at(4 * j + i));
+            for (int i = 0; i < 4; ++i) v[4 * j + i] = ldv(p, o[4 * j + i]);
         }
     }
 };
 
 // op(A) is M x K, op(B) K x N; stored A is M x K (lda = K) or, TA, K x M
 // (lda = M); stored B is K x N (ldb = N) or, TB, N x K (ldb = K). C is M x N.
-template <class Tl, bool TA, bool TB, bool VEC>
+template <class Tl, bool TA, bool TB>
 struct Bf16x3Gemm {
     static constexpr int BM = Tl::BM, BN = Tl::BN, NT = Tl::NT;
     static constexpr int FM = Tl::FM, FN = Tl::FN;
-    using SA = OpStage<BM, NT, !TA, VEC>;
-    using SB = OpStage<BN, NT, TB, VEC>;
+    // PAIR: both operands are staged in 4 x 4 blocks and each has half as many
+    // as the workgroup has lanes (64 x 64 tiles of A^T B): the lower half of
+    // the workgroup then stages A and the upper half B, every lane one block
+    // with 128-bit loads (blocks half as wide, on all lanes for both
+    // operands, halve the bytes per load).
+    static constexpr bool PAIR = TA && !TB && BM == BN && BM * BK / 16 * 2 == NT;
+    template <bool IN, bool EW>
+    using StageA = OpStage<BM, PAIR ? NT / 2 : NT, !TA, IN, EW>;
+    template <bool IN, bool EW>
+    using StageB = OpStage<BN, PAIR ? NT / 2 : NT, TB, IN, EW>;
 
     // One 16-k step of MFMAs on stage `st`: for every 32 x 32 block,
     // acc += lo_a hi_b, then hi_a lo_b, then hi_a hi_b (small terms first).
@@ -379,14 +453,11 @@ struct Bf16x3Gemm {
 
     // Step 0 of stage st with the next stage's split and LDS stores (into nx)
     // between its MFMAs: piece P follows MFMAs [P NM / NP, (P + 1) NM / NP)
-    // behind a scheduling fence, and is followed by the loads (stage bases an,
-    // bn) that refill its registers.
-    __device__ static __forceinline__ void step0_fused(const __bf16 *st, __bf16 *nx, SA &ga, SB &gb,
-                                                       const float *an, const float *bn,
-                                                       const unsigned (&oa)[SA::NLD],
-                                                       const unsigned (&ob)[SB::NLD], int wm,
-                                                       int wn, int lane, int tid,
-                                                       f32x16 (&acc)[FM][FN]) {
+    // behind a scheduling fence, and is followed by the loads that refill its
+    // registers. piece(P): store and refill.
+    template <int NP, class F>
+    __device__ static __forceinline__ void step0_fused(const __bf16 *st, int wm, int wn, int lane,
+                                                       f32x16 (&acc)[FM][FN], F &&piece) {
         const int l32 = lane & 31, koff = 8 * (lane >> 5);
         bf16x8 ah[FM], al[FM], bh[FN], bl[FN];
 #pragma unroll
@@ -401,37 +472,29 @@ struct Bf16x3Gemm {
             bh[fn] = *reinterpret_cast<const bf16x8 *>(st + off);
             bl[fn] = *reinterpret_cast<const bf16x8 *>(st + Tl::B_PLANE + off);
         }
-        constexpr int NPA = SA::NPIECE, NP = NPA + SB::NPIECE, NM = FM * FN * 3;
+        constexpr int NM = FM * FN * 3;
         static_for<0, NP>([&](auto pc) {
             constexpr int P = decltype(pc)::value;
             static_for<P * NM / NP, (P + 1) * NM / NP>([&](auto mc) {
                 mfma_rr<decltype(mc)::value>(ah, al, bh, bl, acc);
             });
-            if constexpr (P < NPA) {
-                ga.template store_piece<P>(nx, nx + Tl::A_PLANE, tid);
-                ga.template load_after_piece<P>(an, oa, tid);
-            } else {
-                gb.template store_piece<P - NPA>(nx + 2 * Tl::A_PLANE,
-                                                 nx + 2 * Tl::A_PLANE + Tl::B_PLANE, tid);
-                gb.template load_after_piece<P - NPA>(bn, ob, tid);
-            }
+            piece(pc);
             __builtin_amdgcn_sched_barrier(0);
         });
     }
 
     // One output tile over k in [0, K) (A, B positioned at that range's
-    // start). INTERIOR: the tile lies inside M x N and K > 0, so no store
-    // and no load of a whole stage needs a bounds check. KTAIL (INTERIOR
-    // only): K is not a whole number of stages, and the last stage's loads
-    // are guarded (zero fill past K); every other stage runs the interior
-    // loop. EPI: what the epilogue stores (bmb::Epi; EPI_PARTIAL: the raw
+    // start). INTERIOR: the tile lies inside M x N. TAIL: K need not be a
+    // whole number of stages (a last stage of fewer k is filled with zeros).
+    // EPI: what the epilogue stores (bmb::Epi; EPI_PARTIAL: the raw
     // sums). C's rows (and those of ep.act, ep.pre) are ldc floats apart.
     // KS > 1: the workgroup is KS k-slices of NT lanes (bf16x3_ks_k); this
     // slice's stages are at smem, K is its range's length (<= 0: none of its
     // stages holds data) and every slice runs kloop stages, so that all of
     // them meet at the same barriers. The slices' sums are then added in LDS,
     // in slice order, and slice 0 runs the epilogue.
-    template <bool INTERIOR, int EPI, bool KTAIL = false, int KS = 1>
+    // EW: M, N or K may be below MIN_DIM (not INTERIOR; see OpStage).
+    template <bool INTERIOR, int EPI, bool TAIL, int KS = 1, bool EW = false>
     __device__ static __forceinline__ void run(int M, int N, int K, int lda, int ldb, float alpha,
                                                const float *__restrict__ A,
                                                const float *__restrict__ B, float beta, float *C,
@@ -450,32 +513,47 @@ struct Bf16x3Gemm {
                 for (int r = 0; r < 16; ++r) acc[fi][fn][r] = 0.0f;
 
         const int nkt = KS > 1 ? kloop : (K + BK - 1) / BK;
+        using SA = StageA<INTERIOR, EW>;
+        using SB = StageB<INTERIOR, EW>;
         SA ga;
         SB gb;
-        unsigned oa[SA::NLD], ob[SB::NLD];
-        if (INTERIOR) {
-            SA::offsets(oa, lda, tid);
-            SB::offsets(ob, ldb, tid);
-        }
-        // Stage kt's bases (uniform): the (row 0, k 0) element of each tile.
+        // PAIR: this half's operand in ga (uniform over a wave).
+        const bool up = PAIR && __builtin_amdgcn_readfirstlane(tid) >= NT / 2;
+        const int stid = PAIR ? tid % (NT / 2) : tid;
+        const int lda1 = up ? ldb : lda, a0 = up ? n0 : m0;
+        ga.setup(up ? N : M, lda1, a0, stid);
+        if (!PAIR) gb.setup(N, ldb, n0, tid);
+        // Stage kt's first elements (uniform).
         auto a_at = [&](int kt) {
-            return TA ? A + (size_t)kt * BK * lda + m0 : A + (size_t)m0 * lda + (size_t)kt * BK;
+            const size_t r = ga.row0(a0), k = (size_t)kt * BK;
+            return (up ? B : A) + (TA ? k * lda1 + r : r * lda1 + k);
         };
         auto b_at = [&](int kt) {
-            return TB ? B + (size_t)n0 * ldb + (size_t)kt * BK : B + (size_t)kt * BK * ldb + n0;
+            const size_t r = gb.row0(n0), k = (size_t)kt * BK;
+            return TB ? B + r * ldb + k : B + k * ldb + r;
         };
         auto load = [&](int kt) {
-            if (INTERIOR && !(KTAIL && kt == nkt - 1)) {
-                ga.load_interior(a_at(kt), oa, tid);
-                gb.load_interior(b_at(kt), ob, tid);
+            const int rem = K - kt * BK;
+            if (EW) {
+                const size_t k = (size_t)kt * BK;
+                ga.load_single((up ? B : A) + (TA ? k * lda1 : k), up ? N : M, lda1, a0, rem,
+                               stid);
+                if (!PAIR) gb.load_single(B + (TB ? k : k * ldb), N, ldb, n0, rem, tid);
+            } else if (!TAIL || rem >= BK) {
+                ga.load(operand(a_at(kt)), stid);
+                if (!PAIR) gb.load(operand(b_at(kt)), tid);
+            } else if (rem > 0) {
+                ga.load_tail(operand(a_at(kt) - (TA ? 0 : 4)), lda1, rem, stid);
+                if (!PAIR) gb.load_tail(operand(b_at(kt) - (TB ? 4 : 0)), ldb, rem, tid);
             } else {
-                ga.load_guarded(A, M, K, lda, m0, kt * BK, tid);
-                gb.load_guarded(B, N, K, ldb, n0, kt * BK, tid);
+                ga.zero();
+                if (!PAIR) gb.zero();
             }
         };
         auto store = [&](__bf16 *st) {
-            ga.store(st, st + Tl::A_PLANE, tid);
-            gb.store(st + 2 * Tl::A_PLANE, st + 2 * Tl::A_PLANE + Tl::B_PLANE, tid);
+            __bf16 *sa = st + (up ? 2 * Tl::A_PLANE : 0);
+            ga.store(sa, sa + Tl::A_PLANE, stid);
+            if (!PAIR) gb.store(st + 2 * Tl::A_PLANE, st + 2 * Tl::A_PLANE + Tl::B_PLANE, tid);
         };
         if (nkt > 0) {
             load(0);
@@ -483,18 +561,35 @@ struct Bf16x3Gemm {
             if (nkt > 1) load(1);
         }
         __syncthreads();
+        // Stages with a next stage to store and a whole one after it to load,
+        // two per turn where the LDS addresses of both stages are in reach of
+        // constant offsets (no address arithmetic is left; the 256 x 256
+        // tile's 128 KB would need a second set of address registers, which
+        // spilled 24-34 of them).
+        constexpr int UNROLL = Tl::SMEM_BYTES <= 98304 ? 2 : 1;
         int kt0 = 0;
-        if (INTERIOR) {
-            // Stages with a next stage to store and a whole stage after it to
-            // load (KTAIL: the last stage is loaded by the loop below).
-            for (; kt0 + 2 < nkt - (KTAIL ? 1 : 0); ++kt0) {
-                const __bf16 *st = smem + (kt0 & 1) * Tl::STAGE;
-                step0_fused(st, smem + ((kt0 + 1) & 1) * Tl::STAGE, ga, gb, a_at(kt0 + 2),
-                            b_at(kt0 + 2), oa, ob, wm, wn, lane, tid, acc);
+        for (const int whole = EW ? 0 : K / BK; kt0 + 1 + UNROLL < whole; kt0 += UNROLL)
+            static_for<0, UNROLL>([&](auto uc) {
+                const int kt = kt0 + uc, h = UNROLL == 2 ? (int)uc : kt & 1;
+                const __bf16 *st = smem + h * Tl::STAGE;
+                __bf16 *nx = smem + (1 - h) * Tl::STAGE, *na = nx + (up ? 2 * Tl::A_PLANE : 0);
+                const auto an = operand(a_at(kt + 2)), bn = operand(b_at(kt + 2));
+                constexpr int NPA = SA::NPIECE;
+                constexpr int NP = NPA + (PAIR ? 0 : SB::NPIECE);
+                step0_fused<NP>(st, wm, wn, lane, acc, [&](auto pc) {
+                    constexpr int P = decltype(pc)::value;
+                    if constexpr (P < NPA) {
+                        ga.template store_piece<P>(na, na + Tl::A_PLANE, stid);
+                        ga.template load_after_piece<P>(an, stid);
+                    } else {
+                        gb.template store_piece<P - NPA>(nx + 2 * Tl::A_PLANE,
+                                                         nx + 2 * Tl::A_PLANE + Tl::B_PLANE, tid);
+                        gb.template load_after_piece<P - NPA>(bn, tid);
+                    }
+                });
                 step(st, 1, wm, wn, lane, acc);
                 __syncthreads();
-            }
-        }
+            });
         for (int kt = kt0; kt < nkt; ++kt) {
             const __bf16 *st = smem + (kt & 1) * Tl::STAGE;
             step(st, 0, wm, wn, lane, acc);
@@ -603,18 +698,17 @@ struct Bf16x3Gemm {
 // when TA, K otherwise), B (at least K when TB, N otherwise) and C (at least
 // N), so that a block of rows and columns of a larger problem (its operands
 // offset to its first row and column) runs as a problem of its own.
-// KT: K is not a whole number of stages; interior tiles then run the
-// interior loop with a guarded last stage (Bf16x3Gemm::run's KTAIL). A
-// separate instantiation: the extra path costs the 256 x 256 kernels about a
-// dozen spilled registers, which the other shapes need not pay.
-template <class Tl, bool TA, bool TB, bool VEC, int EPI, bool KT = false>
+// KT: K is not a whole number of stages. (A separate instantiation: the last
+// stage's loads cost the 256 x 256 kernels spilled registers, which the other
+// shapes need not pay.)
+template <class Tl, bool TA, bool TB, int EPI, bool KT>
 __global__ __launch_bounds__(Tl::NT) void bf16x3_k(int M, int N, int K, int kchunk, float alpha,
                                                    const float *__restrict__ A, int lda,
                                                    const float *__restrict__ B, int ldb,
                                                    float beta, float *C, int ldc, int tiles_m,
                                                    int tiles_n, bmb::EpiArgs ep) {
     extern __shared__ __bf16 lds[];
-    using G = Bf16x3Gemm<Tl, TA, TB, VEC>;
+    using G = Bf16x3Gemm<Tl, TA, TB>;
     int tm, tn;
     bmb::group_tile(bmb::xcd_remap(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, 8, tm, tn);
     const int m0 = tm * Tl::BM, n0 = tn * Tl::BN;
@@ -623,67 +717,99 @@ __global__ __launch_bounds__(Tl::NT) void bf16x3_k(int M, int N, int K, int kchu
     const float *Bk = TB ? B + kb : B + (size_t)kb * ldb;
     float *Cs = EPI == bmb::EPI_PARTIAL ? C + (size_t)blockIdx.y * M * N : C;
     const int ldcs = EPI == bmb::EPI_PARTIAL ? N : ldc;
-    if (m0 + Tl::BM <= M && n0 + Tl::BN <= N && klen > 0 && klen % BK == 0)
-        G::template run<true, EPI>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0, n0,
-                                   lds, ep);
-    else if (KT && m0 + Tl::BM <= M && n0 + Tl::BN <= N && klen > 0)
-        G::template run<true, EPI, true>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0,
-                                         n0, lds, ep);
+    if (m0 + Tl::BM <= M && n0 + Tl::BN <= N)
+        G::template run<true, EPI, KT>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0, n0,
+                                       lds, ep);
     else
-        G::template run<false, EPI>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0, n0,
-                                    lds, ep);
+        G::template run<false, EPI, KT>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0,
+                                        n0, lds, ep);
 }
 
-// The same tile as KS k-slices of Tl::NT lanes each (any epilogue but a
-// split-K partial: it never splits). Every slice runs per = ceil(stages / KS)
-// stages, slice s those from s * per on, in its own KS-th of the LDS, and the
-// slices' sums meet in LDS (Bf16x3Gemm::run). For problems with too few
-// output tiles to fill the device, where split-K would need a second launch
-// for its reduce. A slice of an interior tile whose range is `per` whole
-// stages takes the unguarded loop, the others the guarded one (both loops
-// pass the same number of barriers).
-template <class Tl, bool TA, bool TB, bool VEC, int EPI, int KS>
-__global__ __launch_bounds__(Tl::NT * KS) void bf16x3_ks_k(int M, int N, int K, float alpha,
+// The same tile as KS k-slices of Tl::NT lanes each: every slice runs per =
+// ceil(stages / KS) stages of the workgroup's K range, slice s those from
+// s * per on, in its own KS-th of the LDS, and the slices' sums meet in LDS
+// (Bf16x3Gemm::run). For problems with too few output tiles to fill the
+// device, where split-K alone would need a second launch for its reduce or
+// many more ranges (and partials) for the same number of waves.
+// KT: some slice's range is not `per` whole stages.
+template <class Tl, bool TA, bool TB, int EPI, int KS, bool KT>
+__global__ __launch_bounds__(Tl::NT * KS) void bf16x3_ks_k(int M, int N, int K, int kchunk,
+                                                           float alpha,
                                                            const float *__restrict__ A, int lda,
                                                            const float *__restrict__ B, int ldb,
                                                            float beta, float *C, int ldc,
                                                            int tiles_m, int tiles_n,
                                                            bmb::EpiArgs ep) {
     extern __shared__ __bf16 lds[];
-    using G = Bf16x3Gemm<Tl, TA, TB, VEC>;
+    using G = Bf16x3Gemm<Tl, TA, TB>;
     int tm, tn;
     bmb::group_tile(bmb::xcd_remap(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, 8, tm, tn);
     const int m0 = tm * Tl::BM, n0 = tn * Tl::BN;
-    const int slice = (int)(threadIdx.x / Tl::NT);
-    const int per = ((K + BK - 1) / BK + KS - 1) / KS;
-    const int kb = slice * per * BK;
-    const int klen = min(K - kb, per * BK);  // <= 0: a slice past K (zero stages of data)
-    const float *Ak = TA ? A + (size_t)min(kb, K) * lda : A + min(kb, K);
-    const float *Bk = TB ? B + min(kb, K) : B + (size_t)min(kb, K) * ldb;
+    const int kr = blockIdx.y * kchunk, kend = min(K, kr + kchunk);
+    // (Uniform over a wave, which the compiler cannot see; the descriptors of
+    // the staging loads need it in a scalar register.)
+    const int slice = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / Tl::NT));
+    const int per = ((kend - kr + BK - 1) / BK + KS - 1) / KS;
+    const int kb = min(kr + slice * per * BK, kend);
+    const int klen = min(kend - kb, per * BK);  // 0: a slice past the range
+    const float *Ak = TA ? A + (size_t)kb * lda : A + kb;
+    const float *Bk = TB ? B + kb : B + (size_t)kb * ldb;
+    float *Cs = EPI == bmb::EPI_PARTIAL ? C + (size_t)blockIdx.y * M * N : C;
+    const int ldcs = EPI == bmb::EPI_PARTIAL ? N : ldc;
     __bf16 *st = lds + (size_t)slice * 2 * Tl::STAGE;
-    if (m0 + Tl::BM <= M && n0 + Tl::BN <= N && klen == per * BK)
-        G::template run<true, EPI, false, KS>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, C, ldc,
-                                              m0, n0, st, ep, per);
+    if (m0 + Tl::BM <= M && n0 + Tl::BN <= N)
+        G::template run<true, EPI, KT, KS>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs,
+                                             m0, n0, st, ep, per);
     else
-        G::template run<false, EPI, false, KS>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, C, ldc,
-                                               m0, n0, st, ep, per);
+        G::template run<false, EPI, KT, KS>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs,
+                                              m0, n0, st, ep, per);
+}
+
+// Problems with an M, N or K below MIN_DIM, or too large for 32-bit offsets
+// within a tile (part_time): 64 x 64 tiles whose operands are loaded element
+// by element.
+constexpr int MIN_DIM = 4;
+template <bool TA, bool TB, int EPI>
+__global__ __launch_bounds__(TileS::NT) void bf16x3_narrow_k(int M, int N, int K, int kchunk,
+                                                             float alpha,
+                                                             const float *__restrict__ A, int lda,
+                                                             const float *__restrict__ B, int ldb,
+                                                             float beta, float *C, int ldc,
+                                                             int tiles_m, int tiles_n,
+                                                             bmb::EpiArgs ep) {
+    extern __shared__ __bf16 lds[];
+    int tm, tn;
+    bmb::group_tile(bmb::xcd_remap(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, 8, tm, tn);
+    const int kb = blockIdx.y * kchunk, klen = min(K, kb + kchunk) - kb;
+    const float *Ak = TA ? A + (size_t)kb * lda : A + kb;
+    const float *Bk = TB ? B + kb : B + (size_t)kb * ldb;
+    float *Cs = EPI == bmb::EPI_PARTIAL ? C + (size_t)blockIdx.y * M * N : C;
+    Bf16x3Gemm<TileS, TA, TB>::template run<false, EPI, true, 1, true>(
+        M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, EPI == bmb::EPI_PARTIAL ? N : ldc,
+        tm * TileS::BM, tn * TileS::BN, lds, ep);
 }
 
 // ------------------------------------------------------------- host side
 
-// Tile and split choice, the fp32 MFMA planner's time model (mfma_gemm.hip)
-// with this path's own constants: a work item is one output tile over one K
-// range; the device runs cus x occupancy of them per round; a part-filled
-// last round runs each CU's items faster by (held / fit)^PARTIAL_EXP, and a
-// single round that leaves CUs idle runs faster again by
-// (busy CUs / cus)^FILL_EXP; a split adds the partials' round trip and the
-// reduce. The tile rates and PARTIAL_EXP are fitted to a forced sweep on
-// MI355X of every tile x split count below over the GPT-2 shapes and the
-// square sweep N = 512 ... 8192 (810 timed plans): the model's plan is the
-// measured best, or within 3% of it (the sweep's run-to-run spread), on all
-// of them but N = 2048 (5%). The 128 x 256 tile serves the N = 768 and
-// 3072-wide GPT-2 layers with K = 768 or 3072 (4-9% faster than 128 x 128
-// there); a 256 x 128 tile was never chosen and is not built.
+// Tile and split choice. A work item is one output tile over one K range. A
+// CU that holds r items of a tile at once takes
+//   c + d r + stages (a + b r) (1 + mis u)
+// us for them: per 32-k stage a part that residents overlap (a, the latency
+// chain of a stage) and one that they share (b, the CU's LDS, VALU and matrix
+// cores), a prologue c and an epilogue d. u is the share of the staged bytes
+// whose rows are not a multiple of 16 bytes apart. The device runs cus x
+// occupancy items per round; the last, partial round is charged between its
+// mean and its fullest CU. A split adds the partials' round trip, the reduce
+// launch and a term per range (each reduce lane adds its ranges one after
+// the other), every plan its launch and the write of C. The constants are a
+// least-squares fit (on log time) to 10,000 timed plans of 250 problems on
+// one MI355X: every tile x slices x split below over the linear layers of
+// GPTs of width 256-1024 at 64-16384 rows in all three transposes, squares of
+// 192-4608 and random shapes (M, N, K of 64-8192, a third of them odd). On
+// those the model's plan is 1.8% slower than the best measured one on average
+// (5% at the 90th percentile); the model before it, fitted to the GPT-2
+// layers and squares alone, 3.1% (16%), and up to 1.9x on problems of few
+// tiles or short K.
 //
 // Row bands. A tile count just above a whole number of rounds (4097^2 on
 // 256 x 256: 289 tiles on 256 CUs; 6144^2: 576 tiles, 2.25 rounds; the GPT-2
@@ -694,39 +820,33 @@ __global__ __launch_bounds__(Tl::NT * KS) void bf16x3_ks_k(int M, int N, int K, 
 // split) that suits that remainder, typically a smaller tile or a K split
 // that spreads it over every CU.
 struct B3Cand {
-    int bm, bn;
-    double tflops;  // fitted fp32-equivalent TFLOP/s when the device is full of them
-    int ks;         // k-slices per workgroup (bf16x3_ks_k; never split)
+    int bm, bn, ks;  // tile, and k-slices per workgroup (bf16x3_ks_k)
+    double a, b, c, d, mis;
 };
-constexpr B3Cand CANDS[] = {{256, 256, 452.0, 1}, {128, 128, 326.0, 1}, {64, 64, 233.0, 1},
-                            {128, 256, 345.0, 1}, {64, 64, 233.0, 2},  {64, 64, 233.0, 4},
-                            {32, 32, 180.0, 4},   {32, 32, 180.0, 8}};
+constexpr B3Cand CANDS[] = {
+    {256, 256, 1, 0.000, 2.196, 2.90, 2.87, 0.04},
+    {128, 128, 1, 0.253, 0.562, 2.05, 0.26, 0.08},
+    {64, 64, 1, 0.160, 0.213, 1.10, 0.04, 0.16},
+    {128, 256, 1, 0.000, 1.258, 1.93, 1.32, 0.04},
+    {64, 64, 2, 0.159, 0.437, 1.25, 0.00, 0.17},
+    {64, 64, 4, 0.321, 0.746, 0.59, 1.39, 0.24},
+    {32, 32, 4, 0.251, 0.322, 0.96, 0.00, 0.33},
+    {32, 32, 8, 0.317, 0.628, 0.56, 0.77, 0.38},
+};
 constexpr int N_CANDS = 8;
-// A k-sliced workgroup: each slice beyond the first adds KS_OVERHEAD k to its
-// item (its own prologue and the slices' sum in LDS); the 32 x 32 tile only
-// for problems of at most XS_MAX_OUTPUTS outputs, every slice at least
-// MIN_SLICE_K of k. Fitted to a forced sweep of every plan on ten problems
-// of 0.06-1.1 M outputs (the squares 512-2048, 256 x 256 x 4096, 512 x 512
-// x 2048, 384 x 384 x 1000, 128 x 1024 x 8192): the model's plan is the
-// measured best on all but N = 2048 (5%, as before). The k-sliced plans
-// replace split-K plus its reduce at N = 512 (9.5 -> 5.6 us), 768, 1000 and
-// 1024 (19.4 -> 15.0 us); no GPT-2 shape or square above 1024 changes plan.
-constexpr double KS_OVERHEAD = 64.0;
+constexpr int NARROW = N_CANDS;  // bf16x3_narrow_k, planned as the 64 x 64 tile
+// The 32 x 32 tile is only taken up to XS_MAX_OUTPUTS outputs, and every
+// slice keeps at least MIN_SLICE_K of k.
 constexpr long long XS_MAX_OUTPUTS = 1LL << 20;
 constexpr int MIN_SLICE_K = 64;
 // Split counts that are not powers of two fill the device in one round where
-// {2, 4, 8} do not (the GPT-2 weight gradients: 36 tiles of 256 x 256 in 7
-// ranges on 256 CUs, 36 of 128 x 128 in 14 on 512 slots: 18-36% faster). The
-// model undercharges short ranges, so these are only considered when every
-// range keeps MIN_ODD_SPLIT_K of k (a 7-way split of K = 1536, 224 per
-// range, measured 5.5% slower than the 4-way split the model ranked second).
+// {2, 4, 8} do not (36 tiles of 256 x 256 in 7 ranges on 256 CUs).
 constexpr int SPLITS[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
-constexpr int MIN_ODD_SPLIT_K = 512;
-constexpr double PARTIAL_EXP = 0.63;
-constexpr double FILL_EXP = 0.3;
-constexpr double K_OVERHEAD = 96.0;               // per-item prologue/epilogue, in k
-constexpr double PARTIALS_BYTES_PER_S = 1.35e13;  // the partials' round trip
-constexpr double LAUNCH_S = 1.6e-6;               // the reduce launch
+constexpr double LAUNCH_US = 3.3;                  // one launch, timed back to back
+constexpr double C_BYTES_PER_US = 15.5e6;          // the write of C
+constexpr double PARTIALS_BYTES_PER_US = 11.9e6;   // the partials' round trip
+constexpr double REDUCE_US = 1.1, RANGE_US = 0.27;  // the reduce, and each range in it
+constexpr double FULLEST = 0.67;  // a partial round: the weight of its fullest CU
 // A second band: its launch and the drain between the bands. Bands are only
 // tried for K >= MIN_BAND_K, with K ranges of at least MIN_BAND_SPLIT_K in a
 // split remainder band, and taken when modelled 3% faster than one band:
@@ -738,7 +858,7 @@ constexpr double LAUNCH_S = 1.6e-6;               // the reduce launch
 // split ranges the model undercharges; with it, no other GPT-2 or square
 // sweep shape changes plan. Corner plans (below) are tried for
 // K >= MIN_CORNER_K only, the range they were measured on.
-constexpr double BAND_S = 12.0e-6;
+constexpr double BAND_US = 9.0;
 constexpr double BAND_GAIN = 0.97;
 constexpr int MIN_BAND_K = 768;
 constexpr int MIN_CORNER_K = 4096;
@@ -758,11 +878,11 @@ int occupancy_of(Kern kern, int threads, size_t smem) {
 }
 template <class Tl>
 int occupancy_of() {
-    return occupancy_of(bf16x3_k<Tl, false, false, true, bmb::EPI_BLAS>, Tl::NT, Tl::SMEM_BYTES);
+    return occupancy_of(bf16x3_k<Tl, false, false, bmb::EPI_BLAS, false>, Tl::NT, Tl::SMEM_BYTES);
 }
 template <class Tl, int KS>
 int ks_occupancy_of() {
-    return occupancy_of(bf16x3_ks_k<Tl, false, false, true, bmb::EPI_BLAS, KS>, Tl::NT * KS,
+    return occupancy_of(bf16x3_ks_k<Tl, false, false, bmb::EPI_BLAS, KS, false>, Tl::NT * KS,
                         KS * Tl::SMEM_BYTES);
 }
 
@@ -812,14 +932,19 @@ const Device &device_info(int dev) {
     return info[dev];
 }
 
-// Modelled time of an M x N x K band on tile t with K split s ways; false if
-// that split is not allowed (may_split, max_floats caps splits * M * N).
-bool part_time(const Device &dv, int M, int N, int K, int t, int s, bool may_split,
-               long long max_floats, Part &out, double &time) {
+// Modelled time (us) of an M x N x K band on tile t with K split s ways;
+// false if that split is not allowed (may_split, max_floats caps splits * M *
+// N). mis_a, mis_b: the operand's rows are not 16-byte aligned.
+bool part_time(const Device &dv, int M, int N, int K, int t, int s, bool mis_a, bool mis_b,
+               bool may_split, long long max_floats, Part &out, double &time) {
     const B3Cand &c = CANDS[t];
+    // The staging loads' byte offsets within a tile stay below 2^32.
+    if (std::max(c.bm, c.bn) * (long long)K >= 1LL << 30 ||
+        (BK + 1LL) * std::max(M, N) >= 1LL << 30)
+        return false;
     int splits = 1, kchunk = K;
     if (c.ks > 1) {
-        if (s > 1 || K < c.ks * MIN_SLICE_K) return false;
+        if (K / s < c.ks * MIN_SLICE_K) return false;
         if (c.bm == 32 && (long long)M * N > XS_MAX_OUTPUTS) return false;
     }
     if (s > 1) {
@@ -829,58 +954,61 @@ bool part_time(const Device &dv, int M, int N, int K, int t, int s, bool may_spl
         if (kchunk < MIN_SPLIT_K) return false;
         splits = (K + kchunk - 1) / kchunk;
         if (splits < 2 || (long long)splits * M * N > max_floats) return false;
-        if ((s & (s - 1)) != 0 && kchunk < MIN_ODD_SPLIT_K) return false;
+        if (splits != s) return false;  // (another entry of SPLITS)
     }
-    const long long tiles = (long long)bmb::ceil_div(M, c.bm) * bmb::ceil_div(N, c.bn);
-    const long long items = tiles * splits;
+    const double mn = (double)M * N;
+    const long long items =
+        (long long)bmb::ceil_div(M, c.bm) * bmb::ceil_div(N, c.bn) * splits;
     const int occ = dv.occ[t], cus = dv.cus;
-    const long long slots = (long long)cus * occ;
-    const double t_item = 2.0 * c.bm * c.bn * (kchunk + K_OVERHEAD + (c.ks - 1) * KS_OVERHEAD) *
-                          occ / (c.tflops * 1e12 / cus);
-    const long long full = items / slots, rem = items % slots;
-    time = full * t_item;
-    if (rem) {
-        const long long per_cu = (rem + cus - 1) / cus;
-        double last =
-            per_cu < occ ? t_item * pow((double)per_cu / occ, PARTIAL_EXP) : t_item;
-        if (full == 0 && rem < cus) last *= pow((double)rem / cus, FILL_EXP);
-        time += last;
-    }
-    if (splits > 1) time += (splits + 2.0) * M * N * 4.0 / PARTIALS_BYTES_PER_S + LAUNCH_S;
+    const double stages = bmb::ceil_div(bmb::ceil_div(kchunk, BK), c.ks);
+    const double share = (double)c.bm / (c.bm + c.bn);  // of the staged bytes, A's
+    const double mis = 1.0 + c.mis * ((mis_a ? share : 0.0) + (mis_b ? 1.0 - share : 0.0));
+    auto round = [&](double r) { return c.c + c.d * r + stages * (c.a + c.b * r) * mis; };
+    const long long slots = (long long)cus * occ, rem = items % slots;
+    time = (items / slots) * round(occ) + LAUNCH_US + mn * 4.0 / C_BYTES_PER_US;
+    if (rem)
+        time += FULLEST * round((double)((rem + cus - 1) / cus)) +
+                (1.0 - FULLEST) * round((double)rem / cus);
+    if (splits > 1)
+        time += (2.0 * splits + 1.0) * mn * 4.0 / PARTIALS_BYTES_PER_US + REDUCE_US +
+                splits * RANGE_US;
     out = Part{t, splits, kchunk};
     return true;
 }
 
 // The fastest single-band plan of an M x N x K band (split K ranges of at
 // least min_split_k; k-sliced tiles only if ks_ok).
-double best_part(const Device &dv, int M, int N, int K, bool may_split, long long max_floats,
-                 Part &best, int min_split_k = 0, bool ks_ok = false) {
+double best_part(const Device &dv, int M, int N, int K, bool mis_a, bool mis_b, bool may_split,
+                 long long max_floats, Part &best, int min_split_k = 0, bool ks_ok = false) {
     double best_t = -1.0;
-    best = Part{0, 1, K};
+    const bool narrow = std::min({M, N, K}) < MIN_DIM;
+    best = Part{NARROW, 1, K};
     for (int t = 0; t < N_CANDS; ++t)
         for (int s : SPLITS) {
-            if (CANDS[t].ks > 1 && !ks_ok) continue;
+            if ((CANDS[t].ks > 1 && !ks_ok) || (narrow && t != 2)) continue;
             Part p;
             double tm;
-            if (part_time(dv, M, N, K, t, s, may_split, max_floats, p, tm) &&
+            if (part_time(dv, M, N, K, t, s, mis_a, mis_b, may_split, max_floats, p, tm) &&
                 (p.splits == 1 || p.kchunk >= min_split_k) && (best_t < 0 || tm < best_t)) {
                 best_t = tm;
                 best = p;
+                if (narrow) best.tile = NARROW;
             }
         }
+    if (best_t < 0) best_t = 1e12;  // no tile reaches: NARROW, whatever it takes
     return best_t;
 }
 
 // ks_ok: the k-sliced tiles may run the problem (single-band plans only).
-Plan plan_for(int dev, int M, int N, int K, bool may_split, long long max_floats,
-              bool edges_ok, bool ks_ok) {
+Plan plan_for(int dev, int M, int N, int K, bool mis_a, bool mis_b, bool may_split,
+              long long max_floats, bool edges_ok, bool ks_ok) {
     const Device &dv = device_info(dev);
     Plan best{{Part{0, 1, K}, Part{0, 1, K}}, M, N, false};
     const double single_t =
-        best_part(dv, M, N, K, may_split, max_floats, best.part[0], 0, ks_ok);
+        best_part(dv, M, N, K, mis_a, mis_b, may_split, max_floats, best.part[0], 0, ks_ok);
     double best_t = single_t;
     // Two bands: the first whole rounds of one tile, the rest on its own plan.
-    for (int t = 0; K >= MIN_BAND_K && t < N_CANDS; ++t) {
+    for (int t = 0; K >= MIN_BAND_K && std::min(M, N) >= MIN_DIM && t < N_CANDS; ++t) {
         const B3Cand &c = CANDS[t];
         if (c.ks > 1) continue;
         const long long tiles_n = bmb::ceil_div(N, c.bn);
@@ -890,12 +1018,13 @@ Plan plan_for(int dev, int M, int N, int K, bool may_split, long long max_floats
             if (rows <= 0) continue;
             if (rows * c.bm >= M) break;
             const int m1 = (int)(rows * c.bm);
+            if (M - m1 < MIN_DIM) continue;
             Part p0, p1;
             double t0, t1;
-            if (!part_time(dv, m1, N, K, t, 1, false, 0, p0, t0)) continue;
-            t1 = best_part(dv, M - m1, N, K, may_split, max_floats, p1, MIN_BAND_SPLIT_K);
-            if (t1 < 0) continue;
-            const double tm = t0 + t1 + BAND_S;
+            if (!part_time(dv, m1, N, K, t, 1, mis_a, mis_b, false, 0, p0, t0)) continue;
+            t1 = best_part(dv, M - m1, N, K, mis_a, mis_b, may_split, max_floats, p1,
+                           MIN_BAND_SPLIT_K);
+            const double tm = t0 + t1 + BAND_US;
             if (tm < BAND_GAIN * single_t && tm < best_t) {
                 best_t = tm;
                 best = Plan{{p0, p1}, m1, N, false};
@@ -914,8 +1043,8 @@ Plan plan_for(int dev, int M, int N, int K, bool may_split, long long max_floats
             continue;
         Part p0;
         double t0;
-        if (!part_time(dv, m1, n1, K, t, 1, false, 0, p0, t0)) continue;
-        const double tm = t0 + bmb::edge_model_s(m1, N - n1, M - m1, N, K);
+        if (!part_time(dv, m1, n1, K, t, 1, mis_a, mis_b, false, 0, p0, t0)) continue;
+        const double tm = t0 + 1e6 * bmb::edge_model_s(m1, N - n1, M - m1, N, K);
         if (tm < BAND_GAIN * single_t && tm < best_t) {
             best_t = tm;
             best = Plan{{p0, Part{0, 1, K}}, m1, n1, true};
@@ -926,27 +1055,27 @@ Plan plan_for(int dev, int M, int N, int K, bool may_split, long long max_floats
                         "(%d,%d,%d) model %.1f us (one band %.1f us)\n",
                 M, N, K, best.m1, best.n1, (int)best.edges, best.part[0].tile,
                 best.part[0].splits, best.part[0].kchunk, best.part[1].tile, best.part[1].splits,
-                best.part[1].kchunk, best_t * 1e6, single_t * 1e6);
+                best.part[1].kchunk, best_t, single_t);
     return best;
 }
 
 // Plans are memoised per (device, shape, split permission and cap): the
 // search above costs tens of microseconds, a GEMM call in a training step
 // a few hundred.
-Plan pick(int M, int N, int K, bool may_split, long long max_floats, bool edges_ok,
-          bool ks_ok) {
+Plan pick(int M, int N, int K, bool mis_a, bool mis_b, bool may_split, long long max_floats,
+          bool edges_ok, bool ks_ok) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    using Key = std::tuple<int, int, int, int, bool, long long, bool, bool>;
+    using Key = std::tuple<int, int, int, int, bool, bool, bool, long long, bool, bool>;
     static std::mutex mu;
     static std::map<Key, Plan> memo;
-    const Key key{dev, M, N, K, may_split, max_floats, edges_ok, ks_ok};
+    const Key key{dev, M, N, K, mis_a, mis_b, may_split, max_floats, edges_ok, ks_ok};
     {
         std::lock_guard<std::mutex> lock(mu);
         auto it = memo.find(key);
         if (it != memo.end()) return it->second;
     }
-    const Plan p = plan_for(dev, M, N, K, may_split, max_floats, edges_ok, ks_ok);
+    const Plan p = plan_for(dev, M, N, K, mis_a, mis_b, may_split, max_floats, edges_ok, ks_ok);
     std::lock_guard<std::mutex> lock(mu);
     if (memo.size() > 4096) memo.clear();
     memo.emplace(key, p);
@@ -959,81 +1088,68 @@ struct Strides {
 };
 
 template <class Tl, bool TA, bool TB, int EPI>
-void launch(int M, int N, int K, int kchunk, int splits, float alpha, const float *A,
-            const float *B, float beta, float *C, const Strides &ld, bool vec,
-            hipStream_t stream, bmb::EpiArgs ep) {
+void launch(int M, int N, int K, const Part &p, float alpha, const float *A, const float *B,
+            float beta, float *C, const Strides &ld, hipStream_t stream, bmb::EpiArgs ep) {
     const int tiles_m = bmb::ceil_div(M, Tl::BM), tiles_n = bmb::ceil_div(N, Tl::BN);
-    const dim3 grid(tiles_m * tiles_n, splits);
     auto go = [&](auto kern) {
         bmb::allow_smem(kern, Tl::SMEM_BYTES);
-        bmb::launch(kern, grid, dim3(Tl::NT), Tl::SMEM_BYTES, stream, M, N, K, kchunk, alpha, A,
-                    ld.lda, B, ld.ldb, beta, C, ld.ldc, tiles_m, tiles_n, ep);
+        bmb::launch(kern, dim3(tiles_m * tiles_n, p.splits), dim3(Tl::NT), Tl::SMEM_BYTES, stream,
+                    M, N, K, p.kchunk, alpha, A, ld.lda, B, ld.ldb, beta, C, ld.ldc, tiles_m,
+                    tiles_n, ep);
     };
-    // (A ragged K has the guarded-tail interior kernels for the BLAS and
-    // split-K epilogues; the fused ones run at K = 768 and 3072.)
-    constexpr bool KT_OK = EPI == bmb::EPI_BLAS || EPI == bmb::EPI_PARTIAL;
-    const bool kt = KT_OK && K % BK != 0;
-    if (vec) {
-        if (kt) go(bf16x3_k<Tl, TA, TB, true, EPI, KT_OK>);
-        else go(bf16x3_k<Tl, TA, TB, true, EPI>);
-    } else {
-        if (kt) go(bf16x3_k<Tl, TA, TB, false, EPI, KT_OK>);
-        else go(bf16x3_k<Tl, TA, TB, false, EPI>);
-    }
+    if (K % BK != 0) go(bf16x3_k<Tl, TA, TB, EPI, true>);
+    else go(bf16x3_k<Tl, TA, TB, EPI, false>);
 }
 
-// One band on tile Tl: one launch with the epilogue, or the split partials
-// (EPI_PARTIAL into P) and the shared reduce with the epilogue.
-template <class Tl, bool TA, bool TB, int EPI>
-void run_part(const Part &p, int M, int N, int K, float alpha, const float *A, const float *B,
-              float beta, float *C, const Strides &ld, bool vec, float *P, hipStream_t stream,
-              bmb::EpiArgs ep) {
-    if (p.splits > 1) {
-        launch<Tl, TA, TB, bmb::EPI_PARTIAL>(M, N, K, p.kchunk, p.splits, 1.0f, A, B, 0.0f, P,
-                                             ld, vec, stream, ep);
-        bmb::splitk_reduce_epi(EPI, C, P, p.splits, (long long)M * N, N, ld.ldc, alpha, beta,
-                               stream, ep.bias, ep.act, ep.pre);
-    } else {
-        launch<Tl, TA, TB, EPI>(M, N, K, K, 1, alpha, A, B, beta, C, ld, vec, stream, ep);
-    }
-}
-
-// One k-sliced launch: one workgroup of KS slices per tile.
+// The k-sliced launch: one workgroup of KS slices per tile and K range.
 template <class Tl, bool TA, bool TB, int EPI, int KS>
-void launch_ks(int M, int N, int K, float alpha, const float *A, const float *B, float beta,
-               float *C, const Strides &ld, bool vec, hipStream_t stream, bmb::EpiArgs ep) {
+void launch_ks(int M, int N, int K, const Part &p, float alpha, const float *A, const float *B,
+               float beta, float *C, const Strides &ld, hipStream_t stream, bmb::EpiArgs ep) {
     const int tiles_m = bmb::ceil_div(M, Tl::BM), tiles_n = bmb::ceil_div(N, Tl::BN);
     const size_t smem = (size_t)KS * Tl::SMEM_BYTES;
     auto go = [&](auto kern) {
         bmb::allow_smem(kern, smem);
-        bmb::launch(kern, dim3(tiles_m * tiles_n), dim3(Tl::NT * KS), smem, stream, M, N, K,
-                    alpha, A, ld.lda, B, ld.ldb, beta, C, ld.ldc, tiles_m, tiles_n, ep);
+        bmb::launch(kern, dim3(tiles_m * tiles_n, p.splits), dim3(Tl::NT * KS), smem, stream, M,
+                    N, K, p.kchunk, alpha, A, ld.lda, B, ld.ldb, beta, C, ld.ldc, tiles_m,
+                    tiles_n, ep);
     };
-    if (vec) go(bf16x3_ks_k<Tl, TA, TB, true, EPI, KS>);
-    else go(bf16x3_ks_k<Tl, TA, TB, false, EPI, KS>);
+    if (p.kchunk % (BK * KS) != 0 || K % p.kchunk != 0) go(bf16x3_ks_k<Tl, TA, TB, EPI, KS, true>);
+    else go(bf16x3_ks_k<Tl, TA, TB, EPI, KS, false>);
 }
 
 template <bool TA, bool TB, int EPI>
-void run_band(const Part &p, int M, int N, int K, float alpha, const float *A, const float *B,
-              float beta, float *C, const Strides &ld, bool vec, float *P, hipStream_t stream,
-              bmb::EpiArgs ep) {
-    if (CANDS[p.tile].ks > 1) {
-        // (never planned for a split-K partial)
-        if constexpr (EPI != bmb::EPI_PARTIAL) {
-            switch (p.tile) {
-            case 4: launch_ks<TileS, TA, TB, EPI, 2>(M, N, K, alpha, A, B, beta, C, ld, vec, stream, ep); break;
-            case 5: launch_ks<TileS, TA, TB, EPI, 4>(M, N, K, alpha, A, B, beta, C, ld, vec, stream, ep); break;
-            case 6: launch_ks<TileXS, TA, TB, EPI, 4>(M, N, K, alpha, A, B, beta, C, ld, vec, stream, ep); break;
-            default: launch_ks<TileXS, TA, TB, EPI, 8>(M, N, K, alpha, A, B, beta, C, ld, vec, stream, ep); break;
-            }
-        }
-        return;
-    }
+void launch_tile(int M, int N, int K, const Part &p, float alpha, const float *A, const float *B,
+                 float beta, float *C, const Strides &ld, hipStream_t stream, bmb::EpiArgs ep) {
     switch (p.tile) {
-    case 0: run_part<TileL, TA, TB, EPI>(p, M, N, K, alpha, A, B, beta, C, ld, vec, P, stream, ep); break;
-    case 1: run_part<TileM, TA, TB, EPI>(p, M, N, K, alpha, A, B, beta, C, ld, vec, P, stream, ep); break;
-    case 2: run_part<TileS, TA, TB, EPI>(p, M, N, K, alpha, A, B, beta, C, ld, vec, P, stream, ep); break;
-    default: run_part<TileT, TA, TB, EPI>(p, M, N, K, alpha, A, B, beta, C, ld, vec, P, stream, ep); break;
+    case 0: launch<TileL, TA, TB, EPI>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 1: launch<TileM, TA, TB, EPI>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 2: launch<TileS, TA, TB, EPI>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 3: launch<TileT, TA, TB, EPI>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 4: launch_ks<TileS, TA, TB, EPI, 2>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 5: launch_ks<TileS, TA, TB, EPI, 4>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 6: launch_ks<TileXS, TA, TB, EPI, 4>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 7: launch_ks<TileXS, TA, TB, EPI, 8>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    default:
+        bmb::launch(bf16x3_narrow_k<TA, TB, EPI>,
+                    dim3(bmb::ceil_div(M, TileS::BM) * bmb::ceil_div(N, TileS::BN), p.splits),
+                    dim3(TileS::NT), TileS::SMEM_BYTES, stream, M, N, K, p.kchunk, alpha, A,
+                    ld.lda, B, ld.ldb, beta, C, ld.ldc, bmb::ceil_div(M, TileS::BM),
+                    bmb::ceil_div(N, TileS::BN), ep);
+    }
+}
+
+// One band: one launch with the epilogue, or the split partials (EPI_PARTIAL
+// into P) and the shared reduce with the epilogue.
+template <bool TA, bool TB, int EPI>
+void run_band(const Part &p, int M, int N, int K, float alpha, const float *A, const float *B,
+              float beta, float *C, const Strides &ld, float *P, hipStream_t stream,
+              bmb::EpiArgs ep) {
+    if (p.splits > 1) {
+        launch_tile<TA, TB, bmb::EPI_PARTIAL>(M, N, K, p, 1.0f, A, B, 0.0f, P, ld, stream, ep);
+        bmb::splitk_reduce_epi(EPI, C, P, p.splits, (long long)M * N, N, ld.ldc, alpha, beta,
+                               stream, ep.bias, ep.act, ep.pre);
+    } else {
+        launch_tile<TA, TB, EPI>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep);
     }
 }
 
@@ -1041,9 +1157,9 @@ void run_band(const Part &p, int M, int N, int K, float alpha, const float *A, c
 // partials reuse P after the first band's reduce has read it).
 template <bool TA, bool TB, int EPI>
 void run_plan(const Plan &p, int M, int N, int K, float alpha, const float *A, const float *B,
-              float beta, float *C, bool vec, float *P, hipStream_t stream, bmb::EpiArgs ep) {
+              float beta, float *C, float *P, hipStream_t stream, bmb::EpiArgs ep) {
     const Strides ld{TA ? M : K, TB ? K : N, N};
-    run_band<TA, TB, EPI>(p.part[0], p.m1, p.n1, K, alpha, A, B, beta, C, ld, vec, P, stream, ep);
+    run_band<TA, TB, EPI>(p.part[0], p.m1, p.n1, K, alpha, A, B, beta, C, ld, P, stream, ep);
     if (p.edges) {
         bmb::gemm_edges(true, M, N, K, p.m1, p.n1, alpha, A, ld.lda, B, ld.ldb, beta, C, ld.ldc,
                         P, stream);
@@ -1056,10 +1172,8 @@ void run_plan(const Plan &p, int M, int N, int K, float alpha, const float *A, c
     if (e1.pre) e1.pre += r * N;
     // A band of rows starts r rows (TA: r columns of the stored K x M) in.
     const float *A1 = TA ? A + r : A + r * K;
-    // 16-byte loads of the band need its first row aligned as well.
-    const bool vec1 = vec && (((uintptr_t)A1 & 15) == 0);
-    run_band<TA, TB, EPI>(p.part[1], M - p.m1, N, K, alpha, A1, B, beta, C + r * N, ld, vec1, P,
-                          stream, e1);
+    run_band<TA, TB, EPI>(p.part[1], M - p.m1, N, K, alpha, A1, B, beta, C + r * N, ld, P, stream,
+                          e1);
 }
 
 long long partial_floats(const Plan &p, int M, int N, int K) {
@@ -1087,26 +1201,26 @@ bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const 
                       long long fixed_floats) {
     if (M <= 0 || N <= 0) return true;
     const bmb::EpiArgs ep{bias, act, pre};
-    const int a_contig = ta ? M : K, b_contig = tb ? K : N;
-    const bool vec = a_contig % 4 == 0 && b_contig % 4 == 0 && (((uintptr_t)A & 15) == 0) &&
-                     (((uintptr_t)B & 15) == 0);
     const bool may_split = fixed != nullptr || !bmb::stream_capturing(stream);
     const bool edges_ok = !ta && !tb && epi == bmb::EPI_BLAS;
     // (Every epilogue has k-sliced kernels, so a fused linear layer and
     // gemm() plus the separate bias/GELU pass plan a shape alike and give the
     // same bits.)
     const bool ks_ok = true;
-    Plan p = pick(M, N, K, may_split, fixed ? fixed_floats : MAX_SPLIT_FLOATS, edges_ok, ks_ok);
+    const bool mis_a = (ta ? M : K) % 4 != 0 || ((uintptr_t)A & 15) != 0;
+    const bool mis_b = (tb ? K : N) % 4 != 0 || ((uintptr_t)B & 15) != 0;
+    Plan p = pick(M, N, K, mis_a, mis_b, may_split, fixed ? fixed_floats : MAX_SPLIT_FLOATS,
+                  edges_ok, ks_ok);
     float *P = fixed;
     std::optional<bmb::ScratchLease> lease;
     const long long pf = partial_floats(p, M, N, K);
     if (pf > 0 && fixed == nullptr) {
         lease.emplace(bmb::SCRATCH_GEMM, (size_t)pf * sizeof(float), stream);
         P = static_cast<float *>(lease->get());
-        if (P == nullptr) p = pick(M, N, K, false, 0, edges_ok, ks_ok);  // no scratch: no split
+        if (P == nullptr) p = pick(M, N, K, mis_a, mis_b, false, 0, edges_ok, ks_ok);  // no scratch: no split
     }
 #define BMB_B3(TA_, TB_, EPI_)                                                              \
-    run_plan<TA_, TB_, EPI_>(p, M, N, K, alpha, A, B, beta, C, vec, P, stream, ep);         \
+    run_plan<TA_, TB_, EPI_>(p, M, N, K, alpha, A, B, beta, C, P, stream, ep);              \
     return true;
     if (epi == bmb::EPI_BLAS) {
         if (!ta && !tb) { BMB_B3(false, false, bmb::EPI_BLAS) }

@@ -637,6 +637,32 @@ def test_k_sliced_tiles(gpu, shape, trans, capfd, monkeypatch):
     assert e3 < bound, (e3, bound)
 
 
+# The bf16x3 kernels' edges: a dimension below 4 (elements loaded one by one);
+# rows that end inside a 4-row block, or K inside a 4-k chunk (loaded from
+# further back and shifted into place), at a multiple of 4 that is no whole
+# tile or stage, and one past one; k-slices of a split K.
+EDGE_SHAPES = [(300, 3, 130), (2, 260, 64), (130, 67, 3), (1, 1, 1), (3, 2, 1000),
+               (4, 4, 4), (131, 94, 1001), (257, 66, 2051), (607, 1858, 95), (516, 388, 36),
+               (64, 1024, 4096), (289, 127, 3970), (1291, 1023, 260)]
+
+
+@pytest.mark.parametrize("trans", TRANS, ids=_tag)
+@pytest.mark.parametrize("shape", EDGE_SHAPES, ids=lambda s: "%dx%dx%d" % s)
+def test_edges(gpu, shape, trans):
+    M, N, K = shape
+    ta, tb = trans
+    A = O.fill_xorshift(M * K, 0x1357)
+    B = O.fill_xorshift(K * N, 0x2468)
+    C0 = O.fill_xorshift(M * N, 0x369C)
+    dA, dB, C = dev(A), dev(B), Guarded(M * N, fill=C0)
+    print("gemm edges %s %dx%dx%d" % (_tag(trans), M, N, K), flush=True)
+    bmb.gemm(ta, tb, M, N, K, 0.75, dA.data_ptr(), dB.data_ptr(), 1.25, C.ptr)
+    sync("gemm edges")
+    e3, bound = bf16x3_err(C.get(), ta, tb, M, N, K, 0.75, A, B, 1.25, C0)
+    assert e3 < bound, (e3, bound)
+    assert C.ok()
+
+
 # Shapes drawn at random (fixed seed), run through whatever plan each planner
 # picks for them -- whole tiles, k-sliced workgroups, split-K, row bands,
 # corner plans -- in both arithmetic modes and all four transposes. C sits
