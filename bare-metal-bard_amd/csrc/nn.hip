@@ -62,6 +62,30 @@ inline unsigned grid_for(long long items) {
     return (unsigned)((items + NT - 1) / NT);
 }
 
+// Columns c..c+3 of a row of C: whole, or (RAG) those of them that exist, the
+// others as `fill`.
+template <bool RAG>
+__device__ __forceinline__ float4 ld_cols(const float *row, int c, int C, float fill) {
+    if (!RAG || (c >= 0 && c + 3 < C)) return ldu4(row + c);
+    float4 v = make_float4(fill, fill, fill, fill);
+    if (c + 0 >= 0 && c + 0 < C) v.x = row[c + 0];
+    if (c + 1 >= 0 && c + 1 < C) v.y = row[c + 1];
+    if (c + 2 >= 0 && c + 2 < C) v.z = row[c + 2];
+    if (c + 3 >= 0 && c + 3 < C) v.w = row[c + 3];
+    return v;
+}
+template <bool RAG>
+__device__ __forceinline__ void st_cols(float *row, int c, int C, float4 v) {
+    if (!RAG || (c >= 0 && c + 3 < C)) {
+        stu4(row + c, v);
+        return;
+    }
+    if (c + 0 >= 0 && c + 0 < C) row[c + 0] = v.x;
+    if (c + 1 >= 0 && c + 1 < C) row[c + 1] = v.y;
+    if (c + 2 >= 0 && c + 2 < C) row[c + 2] = v.z;
+    if (c + 3 >= 0 && c + 3 < C) row[c + 3] = v.w;
+}
+
 // ------------------------------------------------------------ row/column maps
 // Row-structured elementwise kernels split each row of width C into float4
 // chunks (the last one may be partial): work item i is row i / C4, columns
@@ -168,11 +192,12 @@ __global__ __launch_bounds__(NT) void encoder_bwd_wte_k(float *dwte, const float
 
 // ------------------------------------------------------------------ layernorm
 // One wave per row, the row held in NCH float4 registers per lane
-// (C <= 256*NCH, C % 4 == 0). Mean first, then the variance about it
-// (src/nn.cu:54-82): biased, eps 1e-5. RES: the row is first formed as
-// res_a + res_b and stored to res_out (residual_forward fused in front: the
-// same one rounding per element, then the same layernorm of the stored sum).
-template <int NCH, bool RES>
+// (C <= 256*NCH; RAG: C % 4 != 0, the row's last chunk is partial). Mean
+// first, then the variance about it (src/nn.cu:54-82): biased, eps 1e-5. RES:
+// the row is first formed as res_a + res_b and stored to res_out
+// (residual_forward fused in front: the same one rounding per element, then
+// the same layernorm of the stored sum).
+template <int NCH, bool RES, bool RAG>
 __global__ __launch_bounds__(NT) void ln_fwd_k(float *out, float *mean, float *rstd,
                                                 const float *inp, const float *weight,
                                                 const float *bias, int N, int C,
@@ -186,11 +211,11 @@ __global__ __launch_bounds__(NT) void ln_fwd_k(float *out, float *mean, float *r
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
-        v[k] = c < C ? ldu4(x + c) : zero4();
+        v[k] = c < C ? ld_cols<RAG>(x, c, C, 0.0f) : zero4();
         if (RES && c < C) {
-            const float4 y = ldu4(res_b + (size_t)row * C + c);
+            const float4 y = ld_cols<RAG>(res_b + (size_t)row * C, c, C, 0.0f);
             v[k] = make_float4(v[k].x + y.x, v[k].y + y.y, v[k].z + y.z, v[k].w + y.w);
-            stu4(res_out + (size_t)row * C + c, v[k]);
+            st_cols<RAG>(res_out + (size_t)row * C, c, C, v[k]);
         }
         s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
     }
@@ -200,7 +225,10 @@ __global__ __launch_bounds__(NT) void ln_fwd_k(float *out, float *mean, float *r
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
         if (c < C) {
-            const float a = v[k].x - mu, b = v[k].y - mu, d = v[k].z - mu, e = v[k].w - mu;
+            const float a = v[k].x - mu;
+            const float b = !RAG || c + 1 < C ? v[k].y - mu : 0.0f;
+            const float d = !RAG || c + 2 < C ? v[k].z - mu : 0.0f;
+            const float e = !RAG || c + 3 < C ? v[k].w - mu : 0.0f;
             q += (a * a + b * b) + (d * d + e * e);
         }
     }
@@ -215,13 +243,14 @@ __global__ __launch_bounds__(NT) void ln_fwd_k(float *out, float *mean, float *r
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
         if (c < C) {
-            const float4 w = ldu4(weight + c), b = ldu4(bias + c);
+            const float4 w = ld_cols<RAG>(weight, c, C, 0.0f);
+            const float4 b = ld_cols<RAG>(bias, c, C, 0.0f);
             float4 o;
             o.x = ((v[k].x - mu) * rs) * w.x + b.x;
             o.y = ((v[k].y - mu) * rs) * w.y + b.y;
             o.z = ((v[k].z - mu) * rs) * w.z + b.z;
             o.w = ((v[k].w - mu) * rs) * w.w + b.w;
-            stu4(y + c, o);
+            st_cols<RAG>(y, c, C, o);
         }
     }
 }
@@ -251,7 +280,7 @@ __global__ __launch_bounds__(NT) void ln_fwd_generic_k(float *out, float *mean, 
     for (int c = lane; c < C; c += 64) y[c] = ((x[c] - mu) * rs) * weight[c] + bias[c];
 }
 
-// Layernorm backward, fused (C % 4 == 0, C <= 256*NCH). A workgroup of
+// Layernorm backward, fused (C <= 256*NCH; RAG: C % 4 != 0). A workgroup of
 // LN_WAVES waves owns rows [blk*rpb, (blk+1)*rpb); each wave takes every
 // LN_WAVES-th of them. Per row (src/nn.cu:85-111):
 //   dinp += rstd * (dxhat - mean(dxhat) - xhat * mean(dxhat * xhat)),
@@ -261,7 +290,7 @@ __global__ __launch_bounds__(NT) void ln_fwd_generic_k(float *out, float *mean, 
 // as partial[blk][0:C] (dweight) and partial[blk][C:2C] (dbias).
 constexpr int LN_WAVES = 8;
 
-template <int NCH>
+template <int NCH, bool RAG>
 __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
     float *dinp, float *partial, const float *dout, const float *inp, const float *weight,
     const float *mean, const float *rstd, int N, int C, int rpb) {
@@ -271,7 +300,7 @@ __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
-        w[k] = c < C ? ldu4(weight + c) : zero4();
+        w[k] = c < C ? ld_cols<RAG>(weight, c, C, 0.0f) : zero4();
         dw[k] = zero4();
         db[k] = zero4();
     }
@@ -289,8 +318,8 @@ __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
             float4 xv = zero4();
             g[k] = zero4();
             if (c < C) {
-                xv = ldu4(x + c);
-                g[k] = ldu4(dy + c);
+                xv = ld_cols<RAG>(x, c, C, mu);  // (xhat 0 past the row's end)
+                g[k] = ld_cols<RAG>(dy, c, C, 0.0f);
             }
             xh[k] = make_float4((xv.x - mu) * rs, (xv.y - mu) * rs, (xv.z - mu) * rs,
                                 (xv.w - mu) * rs);
@@ -306,12 +335,12 @@ __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
         for (int k = 0; k < NCH; ++k) {
             const int c = (k * 64 + lane) * 4;
             if (c < C) {
-                float4 o = ldu4(dx + c);
+                float4 o = ld_cols<RAG>(dx, c, C, 0.0f);
                 o.x += rs * (g[k].x * w[k].x - m1 - xh[k].x * m2);
                 o.y += rs * (g[k].y * w[k].y - m1 - xh[k].y * m2);
                 o.z += rs * (g[k].z * w[k].z - m1 - xh[k].z * m2);
                 o.w += rs * (g[k].w * w[k].w - m1 - xh[k].w * m2);
-                stu4(dx + c, o);
+                st_cols<RAG>(dx, c, C, o);
                 dw[k].x += g[k].x * xh[k].x; dw[k].y += g[k].y * xh[k].y;
                 dw[k].z += g[k].z * xh[k].z; dw[k].w += g[k].w * xh[k].w;
                 db[k].x += g[k].x; db[k].y += g[k].y; db[k].z += g[k].z; db[k].w += g[k].w;
@@ -323,8 +352,13 @@ __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
         if (c < C) {
-            bmb::st4(mine + c, dw[k]);
-            bmb::st4(mine + C + c, db[k]);
+            if (RAG) {
+                st_cols<true>(mine, c, C, dw[k]);
+                st_cols<true>(mine + C, c, C, db[k]);
+            } else {
+                bmb::st4(mine + c, dw[k]);
+                bmb::st4(mine + C + c, db[k]);
+            }
         }
     }
     __syncthreads();
@@ -579,33 +613,44 @@ __global__ __launch_bounds__(NT) void bias_fwd_k(float *out, const float *bias, 
 }
 
 // dlogits[r, i] = (probs[r, i] - [i == target]) * scale for i < V, 0 beyond.
-template <bool VEC>
+// nb workgroups per row (the row is uniform: no division per lane), XB_CH
+// chunks of four columns per lane. RAG: Vp % 4 != 0; a row's chunks then start
+// at the columns that are 16-byte aligned in it, so all but its first and last
+// are still moved by aligned 128-bit accesses (2048 x 50257: 304 -> 153 us,
+// 5.4 TB/s; element by element it ran at half of that).
+constexpr int XB_CH = 4;
+template <bool RAG>
 __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *probs,
-                                                  const int *targets, int V, int Vp, int C4,
-                                                  long long items, float scale) {
-    const long long i = (long long)blockIdx.x * NT + threadIdx.x;
-    if (i >= items) return;
-    const int r = (int)(i / C4), c = (int)(i % C4) * 4;
+                                                  const int *targets, int V, int Vp, int nb,
+                                                  float scale) {
+    const int r = blockIdx.x / nb, part = blockIdx.x % nb;
     const int tgt = targets[r];
-    const float *p = probs + (size_t)r * Vp + c;
-    float *d = dlogits + (size_t)r * Vp + c;
-    if (VEC) {
-        const float4 pv = ldu4(p);
+    const float *p = probs + (size_t)r * Vp;
+    float *d = dlogits + (size_t)r * Vp;
+    const int first = RAG ? -(int)(((size_t)r * Vp) & 3) : 0;
+    float4 v[XB_CH];
+#pragma unroll
+    for (int k = 0; k < XB_CH; ++k) {
+        const int c = first + ((part * XB_CH + k) * NT + (int)threadIdx.x) * 4;
+        if (c < Vp) v[k] = ld_cols<RAG>(p, c, Vp, 0.0f);
+    }
+#pragma unroll
+    for (int k = 0; k < XB_CH; ++k) {
+        const int c = first + ((part * XB_CH + k) * NT + (int)threadIdx.x) * 4;
         float4 o;
-        o.x = c + 0 < V ? (pv.x - (c + 0 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        o.y = c + 1 < V ? (pv.y - (c + 1 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        o.z = c + 2 < V ? (pv.z - (c + 2 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        o.w = c + 3 < V ? (pv.w - (c + 3 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        stu4(d, o);
-    } else {
-        for (int k = 0; k < 4 && c + k < Vp; ++k)
-            d[k] = c + k < V ? (p[k] - (c + k == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+        o.x = c + 0 < V ? (v[k].x - (c + 0 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+        o.y = c + 1 < V ? (v[k].y - (c + 1 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+        o.z = c + 2 < V ? (v[k].z - (c + 2 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+        o.w = c + 3 < V ? (v[k].w - (c + 3 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+        if (c < Vp) st_cols<RAG>(d, c, Vp, o);
     }
 }
 
 // ------------------------------------------------------- softmax + cross-entropy
 // One workgroup of NTHR lanes per row, the row's first V logits held in NCH
-// float4 registers per lane (V <= 4*NTHR*NCH, Vp % 4 == 0): max, then
+// float4 registers per lane (V <= 4*NTHR*NCH; RAG: Vp % 4 != 0, chunks placed
+// as in xent_bwd_k and V <= 4*NTHR*NCH - 3; 2048 x 50257 498 -> 263 us against
+// the three-pass kernel below): max, then
 // exp(x - max) and its sum, then the normalised probabilities -- one read of
 // the logits and one write of the probabilities (src/nn.cu:197-221).
 // exp(x - m) is exp2((x - m) * log2 e) on v_exp_f32.
@@ -625,7 +670,21 @@ __device__ __forceinline__ float block_reduce(float v, float *sh, bool is_max) {
 
 __device__ __forceinline__ float xent_loss(float p) { return -logf(fmaxf(p, 1e-30f)); }
 
-template <int NTHR, int NCH>
+// Columns c..c+3 of a row of C >= 4. RAG: without a branch per element (those
+// made the 16-chunk kernel spill 72 registers): a chunk that runs past the
+// row's end is loaded as the row's last four columns and shifted into place
+// (what follows the last column is unspecified); one that starts before the
+// row reads the end of the row before (c >= 0 in row 0).
+template <bool RAG>
+__device__ __forceinline__ float4 ld_row_end(const float *row, int c, int C) {
+    if (!RAG) return ldu4(row + c);
+    const int at = min(c, C - 4), n = c - at;
+    const float4 v = ldu4(row + at);
+    return make_float4(n == 0 ? v.x : n == 1 ? v.y : n == 2 ? v.z : v.w,
+                       n == 0 ? v.y : n == 1 ? v.z : v.w, n == 0 ? v.z : v.w, v.w);
+}
+
+template <int NTHR, int NCH, bool RAG>
 __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *losses,
                                                         const float *logits, const int *targets,
                                                         int V, int Vp) {
@@ -633,12 +692,17 @@ __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *loss
     const int row = blockIdx.x, tid = threadIdx.x;
     const float *x = logits + (size_t)row * Vp;
     float *p = probs + (size_t)row * Vp;
+    const int first = RAG ? -(int)(((size_t)row * Vp) & 3) : 0;
     float4 v[NCH];
     float m = -INFINITY;
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-        const int c = (k * NTHR + tid) * 4;
-        v[k] = c < V ? ldu4(x + c) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        const int c = first + (k * NTHR + tid) * 4;
+        v[k] = c < V ? ld_row_end<RAG>(x, c, Vp)
+                     : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        if (RAG && c + 0 < 0) v[k].x = -INFINITY;
+        if (RAG && c + 1 < 0) v[k].y = -INFINITY;
+        if (RAG && c + 2 < 0) v[k].z = -INFINITY;
         if (c + 1 >= V) v[k].y = -INFINITY;
         if (c + 2 >= V) v[k].z = -INFINITY;
         if (c + 3 >= V) v[k].w = -INFINITY;
@@ -660,16 +724,25 @@ __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *loss
     const int tgt = targets[row];
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
-        const int c = (k * NTHR + tid) * 4;
+        const int c = first + (k * NTHR + tid) * 4;
         const float4 o = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
-        if (c < Vp) stu4(p + c, o);  // columns in [V, Vp) come out as exp2(-inf) = 0
-        if (tgt >= c && tgt < c + 4 && tgt < V) {
+        if (RAG ? c >= 0 && c + 3 < Vp : c < Vp) stu4(p + c, o);  // columns in [V, Vp) come out as exp2(-inf) = 0
+        if (tgt >= c && tgt < c + 4 && tgt >= 0 && tgt < V) {
             const int j = tgt - c;
             const float pt = j == 0 ? o.x : j == 1 ? o.y : j == 2 ? o.z : o.w;
             losses[row] = xent_loss(pt);
         }
     }
-    for (int c = (NCH * NTHR + tid) * 4; c < Vp; c += NTHR * 4) stu4(p + c, zero4());
+    for (int c = first + (NCH * NTHR + tid) * 4; c < Vp; c += NTHR * 4)
+        if (!RAG || c + 3 < Vp) stu4(p + c, zero4());
+    if (RAG) {
+        // The columns of the row's partial chunks (up to three at each end),
+        // one lane each, from the logits again (with the same arithmetic).
+        const int end = Vp - ((Vp - first) & 3), head = first < 0 ? min(first + 4, Vp) : 0;
+        const int c = tid < 4 ? tid : max(end, head) + tid - 4;
+        if (tid < 4 ? c < head : c < Vp && tid < 8)
+            p[c] = c < V ? __builtin_amdgcn_exp2f(x[c] * LOG2E - ml) * inv : 0.0f;
+    }
     if (tid == 0) {
         if (tgt >= V && tgt < Vp) losses[row] = xent_loss(0.0f);
         if (tgt < 0 || tgt >= Vp) losses[row] = NAN;
@@ -771,9 +844,8 @@ __global__ __launch_bounds__(NT) void sum_k(double *partial, const float *x, lon
 
 // Number of float4 chunks per lane for the register-resident row kernels.
 int row_chunks(int C) {
-    if (C % 4 != 0) return 0;
     const int n = ceil_div(C, 256);
-    return n <= 4 ? n : 0;
+    return n <= 4 ? n : n <= 8 ? 8 : 0;
 }
 
 // Column-sum launch for dout (N, C): G row chunks of rpc rows, chosen from the
@@ -790,12 +862,29 @@ void colsum_finish(float *d0, float *d1, int C0, const float *partial, int G, in
                 C0, partial, G, width);
 }
 
-template <int NCH, bool RES = false>
+template <int NCH, bool RES>
 void ln_fwd_launch(float *out, float *mean, float *rstd, const float *inp, const float *w,
                    const float *b, int N, int C, float *res_out = nullptr,
                    const float *res_b = nullptr) {
-    bmb::launch(ln_fwd_k<NCH, RES>, dim3(ceil_div(N, NT / 64)), dim3(NT), 0, nullptr, out, mean,
-                rstd, inp, w, b, N, C, res_out, res_b);
+    bmb::launch(C % 4 == 0 ? ln_fwd_k<NCH, RES, false> : ln_fwd_k<NCH, RES, true>,
+                dim3(ceil_div(N, NT / 64)), dim3(NT), 0, nullptr, out, mean, rstd, inp, w, b, N, C,
+                res_out, res_b);
+}
+
+// The register-resident forward, if a row fits; false if not.
+template <bool RES>
+bool ln_fwd_rows(float *out, float *mean, float *rstd, const float *inp, const float *w,
+                 const float *b, int N, int C, float *res_out = nullptr,
+                 const float *res_b = nullptr) {
+    switch (row_chunks(C)) {
+        case 1: ln_fwd_launch<1, RES>(out, mean, rstd, inp, w, b, N, C, res_out, res_b); break;
+        case 2: ln_fwd_launch<2, RES>(out, mean, rstd, inp, w, b, N, C, res_out, res_b); break;
+        case 3: ln_fwd_launch<3, RES>(out, mean, rstd, inp, w, b, N, C, res_out, res_b); break;
+        case 4: ln_fwd_launch<4, RES>(out, mean, rstd, inp, w, b, N, C, res_out, res_b); break;
+        case 8: ln_fwd_launch<8, RES>(out, mean, rstd, inp, w, b, N, C, res_out, res_b); break;
+        default: return false;
+    }
+    return true;
 }
 
 template <int NCH>
@@ -803,16 +892,17 @@ void ln_bwd_launch(float *dinp, float *partial, const float *dout, const float *
                    const float *w, const float *mean, const float *rstd, int N, int C, int rpb,
                    int G) {
     const size_t smem = (size_t)LN_WAVES * 2 * C * sizeof(float);
-    bmb::allow_smem(ln_bwd_k<NCH>, smem);
-    bmb::launch(ln_bwd_k<NCH>, dim3(G), dim3(LN_WAVES * 64), smem, nullptr, dinp, partial,
-                dout, inp, w, mean, rstd, N, C, rpb);
+    auto *kern = C % 4 == 0 ? ln_bwd_k<NCH, false> : ln_bwd_k<NCH, true>;
+    bmb::allow_smem(kern, smem);
+    bmb::launch(kern, dim3(G), dim3(LN_WAVES * 64), smem, nullptr, dinp, partial, dout, inp, w,
+                mean, rstd, N, C, rpb);
 }
 
 template <int NTHR, int NCH>
 void xent_launch(float *probs, float *losses, const float *logits, const int *targets, int N,
                  int V, int Vp) {
-    bmb::launch(softmax_xent_k<NTHR, NCH>, dim3(N), dim3(NTHR), 0, nullptr, probs, losses,
-                logits, targets, V, Vp);
+    bmb::launch(Vp % 4 == 0 ? softmax_xent_k<NTHR, NCH, false> : softmax_xent_k<NTHR, NCH, true>,
+                dim3(N), dim3(NTHR), 0, nullptr, probs, losses, logits, targets, V, Vp);
 }
 
 float scalar_result(const float *dptr) {
@@ -828,15 +918,9 @@ void bmb::residual_layernorm_forward(float *res_out, float *ln_out, float *mean,
                                      const float *a, const float *b, const float *weight,
                                      const float *bias, int N, int C) {
     if (N <= 0 || C <= 0) return;
-    switch (row_chunks(C)) {
-        case 1: return ln_fwd_launch<1, true>(ln_out, mean, rstd, a, weight, bias, N, C, res_out, b);
-        case 2: return ln_fwd_launch<2, true>(ln_out, mean, rstd, a, weight, bias, N, C, res_out, b);
-        case 3: return ln_fwd_launch<3, true>(ln_out, mean, rstd, a, weight, bias, N, C, res_out, b);
-        case 4: return ln_fwd_launch<4, true>(ln_out, mean, rstd, a, weight, bias, N, C, res_out, b);
-        default:
-            residual_forward(res_out, a, b, N * C);
-            layernorm_forward(ln_out, mean, rstd, res_out, weight, bias, N, C);
-    }
+    if (ln_fwd_rows<true>(ln_out, mean, rstd, a, weight, bias, N, C, res_out, b)) return;
+    residual_forward(res_out, a, b, N * C);
+    layernorm_forward(ln_out, mean, rstd, res_out, weight, bias, N, C);
 }
 
 extern "C" {
@@ -873,15 +957,9 @@ void encoder_backward(float *dwte, float *dwpe, const float *dout, const int *to
 void layernorm_forward(float *out, float *mean, float *rstd, const float *inp,
                        const float *weight, const float *bias, int N, int C) {
     if (N <= 0 || C <= 0) return;
-    switch (row_chunks(C)) {
-        case 1: ln_fwd_launch<1>(out, mean, rstd, inp, weight, bias, N, C); break;
-        case 2: ln_fwd_launch<2>(out, mean, rstd, inp, weight, bias, N, C); break;
-        case 3: ln_fwd_launch<3>(out, mean, rstd, inp, weight, bias, N, C); break;
-        case 4: ln_fwd_launch<4>(out, mean, rstd, inp, weight, bias, N, C); break;
-        default:
-            bmb::launch(ln_fwd_generic_k, dim3(ceil_div(N, NT / 64)), dim3(NT), 0, nullptr, out,
-                        mean, rstd, inp, weight, bias, N, C);
-    }
+    if (!ln_fwd_rows<false>(out, mean, rstd, inp, weight, bias, N, C))
+        bmb::launch(ln_fwd_generic_k, dim3(ceil_div(N, NT / 64)), dim3(NT), 0, nullptr, out, mean,
+                    rstd, inp, weight, bias, N, C);
 }
 
 void layernorm_backward(float *dinp, float *dweight, float *dbias, const float *dout,
@@ -901,7 +979,8 @@ void layernorm_backward(float *dinp, float *dweight, float *dbias, const float *
             case 1: ln_bwd_launch<1>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
             case 2: ln_bwd_launch<2>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
             case 3: ln_bwd_launch<3>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
-            default: ln_bwd_launch<4>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
+            case 4: ln_bwd_launch<4>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
+            default: ln_bwd_launch<8>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
         }
         colsum_finish(dweight, dbias, C, partial, G, 2 * C);
         return;
@@ -961,12 +1040,13 @@ void bias_backward(float *dbias, const float *dout, int N, int C) {
 void softmax_crossentropy_forward(float *probs, float *losses, const float *logits,
                                   const int *targets, int N, int V, int Vp) {
     if (N <= 0 || V <= 0 || Vp < V) return;
-    if (Vp % 4 == 0) {
-        if (V <= 1024) return xent_launch<256, 1>(probs, losses, logits, targets, N, V, Vp);
-        if (V <= 4096) return xent_launch<256, 4>(probs, losses, logits, targets, N, V, Vp);
-        if (V <= 16384) return xent_launch<1024, 4>(probs, losses, logits, targets, N, V, Vp);
-        if (V <= 32768) return xent_launch<1024, 8>(probs, losses, logits, targets, N, V, Vp);
-        if (V <= 65536) return xent_launch<1024, 16>(probs, losses, logits, targets, N, V, Vp);
+    const int span = Vp % 4 == 0 ? V : V + 3;  // a ragged row's chunks start up to 3 early
+    if (Vp >= 4) {
+        if (span <= 1024) return xent_launch<256, 1>(probs, losses, logits, targets, N, V, Vp);
+        if (span <= 4096) return xent_launch<256, 4>(probs, losses, logits, targets, N, V, Vp);
+        if (span <= 16384) return xent_launch<1024, 4>(probs, losses, logits, targets, N, V, Vp);
+        if (span <= 32768) return xent_launch<1024, 8>(probs, losses, logits, targets, N, V, Vp);
+        if (span <= 65536) return xent_launch<1024, 16>(probs, losses, logits, targets, N, V, Vp);
     }
     bmb::launch(softmax_xent_generic_k, dim3(N), dim3(NT), 0, nullptr, probs, losses, logits,
                 targets, V, Vp);
@@ -975,14 +1055,16 @@ void softmax_crossentropy_forward(float *probs, float *losses, const float *logi
 void crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets,
                                    int N, int V, int Vp, float dloss_scale) {
     if (N <= 0 || Vp <= 0) return;
-    const int C4 = ceil_div(Vp, 4);
-    const long long items = (long long)N * C4;
-    if (Vp % 4 == 0)
-        bmb::launch(xent_bwd_k<true>, dim3(grid_for(items)), dim3(NT), 0, nullptr, dlogits,
-                    probs, targets, V, Vp, C4, items, dloss_scale);
-    else
-        bmb::launch(xent_bwd_k<false>, dim3(grid_for(items)), dim3(NT), 0, nullptr, dlogits,
-                    probs, targets, V, Vp, C4, items, dloss_scale);
+    const int nb = ceil_div(ceil_div(Vp + (Vp % 4 == 0 ? 0 : 3), 4), XB_CH * NT);
+    // Rows per launch: a dispatch holds fewer than 2^32 lanes.
+    const int rows = (int)std::max(1LL, ((1LL << 32) - 1) / NT / nb);
+    for (int r = 0; r < N; r += rows) {
+        const size_t off = (size_t)r * Vp;
+        const bool rag = Vp % 4 != 0;
+        bmb::launch(rag ? xent_bwd_k<true> : xent_bwd_k<false>,
+                    dim3((unsigned)std::min(rows, N - r) * nb), dim3(NT), 0, nullptr,
+                    dlogits + off, probs + off, targets + r, V, Vp, nb, dloss_scale);
+    }
 }
 
 void adamw_update(float *params, float *grads, float *m, float *v, int n, float lr, float beta1,

@@ -78,7 +78,8 @@ def test_encoder(gpu, B, T, C, V):
 
 
 @pytest.mark.parametrize("N,C", [(256, 128), (8192, 768), (37, 1024), (50, 100), (9, 1536),
-                                 (5, 4), (3, 1)])
+                                 (5, 4), (3, 1), (70, 255), (41, 1025), (33, 1599), (19, 2048),
+                                 (6, 2051)])
 def test_layernorm(gpu, N, C):
     r = _rng(2)
     x = _f32(r.standard_normal((N, C)) * 2 + 0.3)
@@ -184,7 +185,9 @@ def test_bias(gpu, N, C):
 
 
 @pytest.mark.parametrize("N,V,Vp", [(256, 65, 128), (64, 50257, 50304), (17, 3000, 3001),
-                                    (5, 70000, 70004), (9, 1, 4), (33, 1000, 1000)])
+                                    (5, 70000, 70004), (9, 1, 4), (33, 1000, 1000),
+                                    (37, 50257, 50257), (9, 1021, 1021), (7, 1022, 1025),
+                                    (5, 65533, 65534), (6, 3, 5), (5, 2, 3)])
 def test_softmax_crossentropy(gpu, N, V, Vp):
     r = _rng(6)
     logits = _f32(r.standard_normal((N, Vp)) * 3)
