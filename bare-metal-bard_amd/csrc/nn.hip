@@ -39,6 +39,15 @@ __device__ __forceinline__ float4 ldu4(const float *p) {
     return v;
 }
 __device__ __forceinline__ void stu4(float *p, float4 v) { __builtin_memcpy(p, &v, sizeof(v)); }
+// The same past the caches. For outputs larger than the 256 MB last-level
+// cache, whose lines would only push out what the next kernels read: at 8192 x
+// 50304 (1.65 GB) the cross-entropy backward took 513 us instead of 532 and the
+// softmax 585 instead of 618; at 4096 x 4096 (67 MB) they took 2-3% longer.
+constexpr size_t STREAM_BYTES = 512u << 20;
+__device__ __forceinline__ void stu4_nt(float *p, float4 v) {
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    __builtin_nontemporal_store(f4{v.x, v.y, v.z, v.w}, reinterpret_cast<f4 *>(p));
+}
 __device__ __forceinline__ float4 zero4() { return make_float4(0.f, 0.f, 0.f, 0.f); }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -141,52 +150,111 @@ __global__ __launch_bounds__(NT) void encoder_bwd_wpe_k(float *dwpe, const float
 }
 
 // dwte[tok, :] += sum over positions j with tokens[j] == tok, j ascending.
-// One wave per position i. A position that is not the first occurrence of
-// its token leaves; the first one gathers every later occurrence in order and
-// owns the update of that wte row, so no two waves touch the same row.
+// One wave per position i (and strip of 256 NCH columns). A position that is
+// not the first occurrence of its token leaves; the first one gathers every
+// occurrence in order and owns the update of that wte row, so no two waves
+// touch the same row. What bounds it is the pass over the ids: a chain of
+// dependent loads where few tokens own many positions, and instructions where
+// most positions are a token's only one. So it takes WTE_IDS ids at a time
+// with 128-bit loads, and only where it finds the token lists the positions in
+// LDS, in ascending order, and loads their rows eight at a time. (64 ids and
+// one row per step took 53 us at 4096 positions of 65 tokens x 384, 88 us at
+// 8192 of 50257 x 768 and 7.3 ms where all 8192 are one token; now 21, 58 and 1200 us.)
+constexpr int WTE_IDS = 1024;
+
+// ids[k] = the lane's ids tokens[j0 + 256 k + 4 lane + 0..3], `other` from
+// position `end` on.
+__device__ __forceinline__ void load_ids(int4 (&ids)[WTE_IDS / 256], const int *tokens, int j0,
+                                         int end, int other, int lane) {
+    const int *p = tokens + j0 + 4 * lane;
+#pragma unroll
+    for (int k = 0; k < WTE_IDS / 256; ++k) {
+        if (j0 + WTE_IDS <= end) {
+            __builtin_memcpy(&ids[k], p + 256 * k, sizeof(int4));
+        } else {
+            const int left = end - (j0 + 4 * lane + 256 * k);
+            ids[k].x = left > 0 ? p[256 * k] : other;
+            ids[k].y = left > 1 ? p[256 * k + 1] : other;
+            ids[k].z = left > 2 ? p[256 * k + 2] : other;
+            ids[k].w = left > 3 ? p[256 * k + 3] : other;
+        }
+    }
+}
+__device__ __forceinline__ bool any_is(const int4 (&ids)[WTE_IDS / 256], int tok) {
+    bool hit = false;
+#pragma unroll
+    for (int k = 0; k < WTE_IDS / 256; ++k)
+        hit |= ids[k].x == tok || ids[k].y == tok || ids[k].z == tok || ids[k].w == tok;
+    return __ballot(hit) != 0;
+}
+
+template <int NCH, bool VEC>
 __global__ __launch_bounds__(NT) void encoder_bwd_wte_k(float *dwte, const float *dout,
                                                          const int *tokens, int N, int C) {
-    const int i = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    __shared__ int found[NT / 64][WTE_IDS];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int i = blockIdx.x * (NT / 64) + wave;
     if (i >= N) return;
-    const int tok = tokens[i];
-    for (int j0 = 0; j0 < i; j0 += 64) {
-        const int j = j0 + lane;
-        if (__ballot(j < i && tokens[j] == tok) != 0) return;
+    const int tok = __builtin_amdgcn_readfirstlane(tokens[i]);
+    int4 ids[WTE_IDS / 256];
+    for (int j0 = 0; j0 < i; j0 += WTE_IDS) {
+        load_ids(ids, tokens, j0, i, ~tok, lane);
+        if (any_is(ids, tok)) return;
     }
-    const bool vec = (C & 3) == 0;
-    float *dst = dwte + (size_t)tok * C;
-    for (int c0 = 0; c0 < C; c0 += 256) {
-        const int c = c0 + lane * 4;
-        float4 s = zero4();
-        for (int j0 = i; j0 < N; j0 += 64) {
-            const int j = j0 + lane;
-            unsigned long long m = __ballot(j < N && tokens[j] == tok);
-            while (m != 0) {
-                const int jj = j0 + __ffsll((long long)m) - 1;
-                m &= m - 1;
-                const float *src = dout + (size_t)jj * C + c;
-                if (vec && c < C) {
-                    const float4 v = ldu4(src);
-                    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-                } else if (!vec) {
-                    if (c + 0 < C) s.x += src[0];
-                    if (c + 1 < C) s.y += src[1];
-                    if (c + 2 < C) s.z += src[2];
-                    if (c + 3 < C) s.w += src[3];
-                }
+    const int c0 = blockIdx.y * 256 * NCH + lane * 4;
+    int *list = found[wave];
+    float4 s[NCH];
+#pragma unroll
+    for (int h = 0; h < NCH; ++h) s[h] = zero4();
+    for (int j0 = i; j0 < N; j0 += WTE_IDS) {
+        load_ids(ids, tokens, j0, N, ~tok, lane);
+        if (!any_is(ids, tok)) continue;
+        int n = 0;
+        const unsigned long long below = (1ULL << lane) - 1;
+#pragma unroll
+        for (int k = 0; k < WTE_IDS / 256; ++k) {
+            const int id[4] = {ids[k].x, ids[k].y, ids[k].z, ids[k].w};
+            int at = n;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned long long m = __ballot(id[e] == tok);
+                at += __popcll(m & below);
+                n += __popcll(m);
             }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (id[e] == tok) list[at++] = j0 + 256 * k + 4 * lane + e;
         }
-        if (vec && c < C) {
-            float4 d = ldu4(dst + c);
-            d.x += s.x; d.y += s.y; d.z += s.z; d.w += s.w;
-            stu4(dst + c, d);
-        } else if (!vec) {
-            if (c + 0 < C) dst[c + 0] += s.x;
-            if (c + 1 < C) dst[c + 1] += s.y;
-            if (c + 2 < C) dst[c + 2] += s.z;
-            if (c + 3 < C) dst[c + 3] += s.w;
+        // The list is this wave's own, and its LDS accesses are in order.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int q = 0; q < n; q += 8) {
+            float4 v[8][NCH];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float *src = dout + (size_t)list[min(q + k, n - 1)] * C;
+#pragma unroll
+                for (int h = 0; h < NCH; ++h)
+                    if (c0 + 256 * h < C) v[k][h] = ld_cols<!VEC>(src, c0 + 256 * h, C, 0.0f);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (q + k < n)
+#pragma unroll
+                    for (int h = 0; h < NCH; ++h) {
+                        s[h].x += v[k][h].x; s[h].y += v[k][h].y;
+                        s[h].z += v[k][h].z; s[h].w += v[k][h].w;
+                    }
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    float *dst = dwte + (size_t)tok * C;
+#pragma unroll
+    for (int h = 0; h < NCH; ++h) {
+        const int c = c0 + 256 * h;
+        if (c >= C) continue;
+        float4 d = ld_cols<!VEC>(dst, c, C, 0.0f);
+        d.x += s[h].x; d.y += s[h].y; d.z += s[h].z; d.w += s[h].w;
+        st_cols<!VEC>(dst, c, C, d);
     }
 }
 
@@ -613,37 +681,35 @@ __global__ __launch_bounds__(NT) void bias_fwd_k(float *out, const float *bias, 
 }
 
 // dlogits[r, i] = (probs[r, i] - [i == target]) * scale for i < V, 0 beyond.
-// nb workgroups per row (the row is uniform: no division per lane), XB_CH
-// chunks of four columns per lane. RAG: Vp % 4 != 0; a row's chunks then start
-// at the columns that are 16-byte aligned in it, so all but its first and last
-// are still moved by aligned 128-bit accesses (2048 x 50257: 304 -> 153 us,
-// 5.4 TB/s; element by element it ran at half of that).
-constexpr int XB_CH = 4;
+// nb workgroups per row (the row is uniform: no division per lane), one chunk
+// of four columns per lane (four chunks: 618 instead of 532 us at 8192 x
+// 50304). RAG: Vp % 4 != 0; a row's chunks then start at the columns that are
+// 16-byte aligned in it, so all but its first and last are still moved by
+// aligned 128-bit accesses (2048 x 50257: 281 -> 133 us). nt: streaming
+// stores, for results that do not fit the last-level cache anyway.
 template <bool RAG>
 __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *probs,
                                                   const int *targets, int V, int Vp, int nb,
-                                                  float scale) {
+                                                  float scale, bool nt) {
     const int r = blockIdx.x / nb, part = blockIdx.x % nb;
     const int tgt = targets[r];
     const float *p = probs + (size_t)r * Vp;
     float *d = dlogits + (size_t)r * Vp;
     const int first = RAG ? -(int)(((size_t)r * Vp) & 3) : 0;
-    float4 v[XB_CH];
-#pragma unroll
-    for (int k = 0; k < XB_CH; ++k) {
-        const int c = first + ((part * XB_CH + k) * NT + (int)threadIdx.x) * 4;
-        if (c < Vp) v[k] = ld_cols<RAG>(p, c, Vp, 0.0f);
-    }
-#pragma unroll
-    for (int k = 0; k < XB_CH; ++k) {
-        const int c = first + ((part * XB_CH + k) * NT + (int)threadIdx.x) * 4;
-        float4 o;
-        o.x = c + 0 < V ? (v[k].x - (c + 0 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        o.y = c + 1 < V ? (v[k].y - (c + 1 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        o.z = c + 2 < V ? (v[k].z - (c + 2 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        o.w = c + 3 < V ? (v[k].w - (c + 3 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-        if (c < Vp) st_cols<RAG>(d, c, Vp, o);
-    }
+    const int c = first + (part * NT + (int)threadIdx.x) * 4;
+    if (c >= Vp) return;
+    const float4 v = ld_cols<RAG>(p, c, Vp, 0.0f);
+    float4 o;
+    o.x = c + 0 < V ? (v.x - (c + 0 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+    o.y = c + 1 < V ? (v.y - (c + 1 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+    o.z = c + 2 < V ? (v.z - (c + 2 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+    o.w = c + 3 < V ? (v.w - (c + 3 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+    if (RAG && (c < 0 || c + 3 >= Vp))
+        st_cols<true>(d, c, Vp, o);
+    else if (nt)
+        stu4_nt(d + c, o);
+    else
+        stu4(d + c, o);
 }
 
 // ------------------------------------------------------- softmax + cross-entropy
@@ -684,7 +750,7 @@ __device__ __forceinline__ float4 ld_row_end(const float *row, int c, int C) {
                        n == 0 ? v.y : n == 1 ? v.z : v.w, n == 0 ? v.z : v.w, v.w);
 }
 
-template <int NTHR, int NCH, bool RAG>
+template <int NTHR, int NCH, bool RAG, bool STREAM>
 __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *losses,
                                                         const float *logits, const int *targets,
                                                         int V, int Vp) {
@@ -726,7 +792,7 @@ __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *loss
     for (int k = 0; k < NCH; ++k) {
         const int c = first + (k * NTHR + tid) * 4;
         const float4 o = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
-        if (RAG ? c >= 0 && c + 3 < Vp : c < Vp) stu4(p + c, o);  // columns in [V, Vp) come out as exp2(-inf) = 0
+        if (RAG ? c >= 0 && c + 3 < Vp : c < Vp) STREAM ? stu4_nt(p + c, o) : stu4(p + c, o);  // columns in [V, Vp) come out as exp2(-inf) = 0
         if (tgt >= c && tgt < c + 4 && tgt >= 0 && tgt < V) {
             const int j = tgt - c;
             const float pt = j == 0 ? o.x : j == 1 ? o.y : j == 2 ? o.z : o.w;
@@ -901,8 +967,12 @@ void ln_bwd_launch(float *dinp, float *partial, const float *dout, const float *
 template <int NTHR, int NCH>
 void xent_launch(float *probs, float *losses, const float *logits, const int *targets, int N,
                  int V, int Vp) {
-    bmb::launch(Vp % 4 == 0 ? softmax_xent_k<NTHR, NCH, false> : softmax_xent_k<NTHR, NCH, true>,
-                dim3(N), dim3(NTHR), 0, nullptr, probs, losses, logits, targets, V, Vp);
+    const bool stream = (size_t)N * Vp * sizeof(float) >= STREAM_BYTES;
+    auto *kern = Vp % 4 == 0 ? (stream ? softmax_xent_k<NTHR, NCH, false, true>
+                                       : softmax_xent_k<NTHR, NCH, false, false>)
+                             : (stream ? softmax_xent_k<NTHR, NCH, true, true>
+                                       : softmax_xent_k<NTHR, NCH, true, false>);
+    bmb::launch(kern, dim3(N), dim3(NTHR), 0, nullptr, probs, losses, logits, targets, V, Vp);
 }
 
 float scalar_result(const float *dptr) {
@@ -950,8 +1020,14 @@ void encoder_backward(float *dwte, float *dwpe, const float *dout, const int *to
         bmb::launch(encoder_bwd_wpe_k<false>, dim3(grid_for(items)), dim3(NT), 0, nullptr,
                     dwpe, dout, B, T, C, C4, items);
     const int N = B * T;
-    bmb::launch(encoder_bwd_wte_k, dim3(ceil_div(N, NT / 64)), dim3(NT), 0, nullptr, dwte, dout,
-                tokens, N, C);
+    auto wte = [&](auto kern, int nch) {
+        bmb::launch(kern, dim3(ceil_div(N, NT / 64), ceil_div(C, 256 * nch)), dim3(NT), 0, nullptr,
+                    dwte, dout, tokens, N, C);
+    };
+    if (C % 4 != 0) wte(encoder_bwd_wte_k<1, false>, 1);
+    else if (C <= 256) wte(encoder_bwd_wte_k<1, true>, 1);
+    else if (C <= 512) wte(encoder_bwd_wte_k<2, true>, 2);
+    else wte(encoder_bwd_wte_k<3, true>, 3);
 }
 
 void layernorm_forward(float *out, float *mean, float *rstd, const float *inp,
@@ -1055,7 +1131,8 @@ void softmax_crossentropy_forward(float *probs, float *losses, const float *logi
 void crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets,
                                    int N, int V, int Vp, float dloss_scale) {
     if (N <= 0 || Vp <= 0) return;
-    const int nb = ceil_div(ceil_div(Vp + (Vp % 4 == 0 ? 0 : 3), 4), XB_CH * NT);
+    const int nb = ceil_div(ceil_div(Vp + (Vp % 4 == 0 ? 0 : 3), 4), NT);
+    const bool nt = (size_t)N * Vp * sizeof(float) >= STREAM_BYTES;
     // Rows per launch: a dispatch holds fewer than 2^32 lanes.
     const int rows = (int)std::max(1LL, ((1LL << 32) - 1) / NT / nb);
     for (int r = 0; r < N; r += rows) {
@@ -1063,7 +1140,7 @@ void crossentropy_softmax_backward(float *dlogits, const float *probs, const int
         const bool rag = Vp % 4 != 0;
         bmb::launch(rag ? xent_bwd_k<true> : xent_bwd_k<false>,
                     dim3((unsigned)std::min(rows, N - r) * nb), dim3(NT), 0, nullptr,
-                    dlogits + off, probs + off, targets + r, V, Vp, nb, dloss_scale);
+                    dlogits + off, probs + off, targets + r, V, Vp, nb, dloss_scale, nt);
     }
 }
 
