@@ -15,9 +15,13 @@ void gemm_bias_nt(int M, int N, int K, const float *A, const float *W, const flo
 
 // C[M,N] = gelu_grad(pre, A[M,K] @ B[K,N]) elementwise: the dX GEMM of the
 // FC projection (gemm(false, false, ...)) followed by gelu_backward
-// (src/gpt.cu:331-337), without storing the product.
-void gemm_gelu_grad_nn(int M, int N, int K, const float *A, const float *B, const float *pre,
-                       float *C);
+// (src/gpt.cu:331-337), without storing the product. Where the plan allows it
+// (bf16x3, K not split), it also leaves partial column sums of C (the bias
+// gradient of the layer before) in colsum, at most gelu_grad_sum_rows(M) rows
+// of N, and returns how many rows; 0 if none.
+inline int gelu_grad_sum_rows(int M) { return (M + 31) / 32 + 4; }
+int gemm_gelu_grad_nn(int M, int N, int K, const float *A, const float *B, const float *pre,
+                      float *C, float *colsum);
 
 // C = alpha * sum_{s < splits} P[s] + beta * C over mn = M * N floats (P is
 // splits x M x N), the splits added in ascending order: the reduce of every
@@ -40,10 +44,11 @@ void splitk_reduce_epi(int epi, float *C, const float *P, int splits, long long 
 // EPI_GELU_GRAD (no transposes). Split-K partials go to `fixed` (at most
 // fixed_floats floats) on any stream, or to leased scratch on the null stream
 // only. Returns false, launching nothing, for an unsupported combination.
+// colsum, colsum_rows (EPI_GELU_GRAD): as in gemm_gelu_grad_nn.
 bool bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const float *A,
                  const float *B, float beta, float *C, hipStream_t stream, int epi,
                  const float *bias, float *act, const float *pre, float *fixed,
-                 long long fixed_floats);
+                 long long fixed_floats, float *colsum = nullptr, int *colsum_rows = nullptr);
 
 // Thin edges of a corner plan (edge_gemm.hip): of an M x N x K problem with
 // row-major A (lda), B (ldb) and C (ldc), C = alpha A B + beta C over rows

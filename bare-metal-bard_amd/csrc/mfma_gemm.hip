@@ -661,7 +661,7 @@ void fp32_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const float *
 void bmb::gemm_bias_nt(int M, int N, int K, const float *A, const float *W, const float *bias,
                        float *C, float *gelu_out) {
     if (fp32_math()) {
-        const bmb::EpiArgs ep{bias, gelu_out, nullptr};
+        const bmb::EpiArgs ep{bias, gelu_out, nullptr, nullptr};
         if (gelu_out != nullptr)
             dispatch<false, true, bmb::EPI_BIAS_GELU>(1, M, N, K, 1.0f, A, 0, W, 0, 0.0f, C, 0,
                                                       nullptr, ep);
@@ -675,15 +675,18 @@ void bmb::gemm_bias_nt(int M, int N, int K, const float *A, const float *W, cons
                      nullptr, nullptr, 0);
 }
 
-void bmb::gemm_gelu_grad_nn(int M, int N, int K, const float *A, const float *B,
-                            const float *pre, float *C) {
+int bmb::gemm_gelu_grad_nn(int M, int N, int K, const float *A, const float *B,
+                           const float *pre, float *C, float *colsum) {
     if (fp32_math()) {
         dispatch<false, false, bmb::EPI_GELU_GRAD>(1, M, N, K, 1.0f, A, 0, B, 0, 0.0f, C, 0,
-                                                   nullptr, bmb::EpiArgs{nullptr, nullptr, pre});
-        return;
+                                                   nullptr,
+                                                   bmb::EpiArgs{nullptr, nullptr, pre, nullptr});
+        return 0;
     }
+    int rows = 0;
     bmb::bf16x3_gemm(false, false, M, N, K, 1.0f, A, B, 0.0f, C, nullptr, bmb::EPI_GELU_GRAD,
-                     nullptr, nullptr, pre, nullptr, 0);
+                     nullptr, nullptr, pre, nullptr, 0, colsum, &rows);
+    return rows;
 }
 
 void bmb::splitk_reduce(float *C, const float *P, int splits, long long mn, int N, float alpha,
@@ -696,7 +699,7 @@ void bmb::splitk_reduce_epi(int epi, float *C, const float *P, int splits, long 
                             int ldc, float alpha, float beta, hipStream_t stream,
                             const float *bias, float *act, const float *pre) {
     const dim3 grid((unsigned)((mn + 1023) / 1024)), block(256);
-    const bmb::EpiArgs ep{bias, act, pre};
+    const bmb::EpiArgs ep{bias, act, pre, nullptr};
     switch (epi) {
     case bmb::EPI_BIAS:
         bmb::launch(bmb::splitk_reduce_k<bmb::EPI_BIAS>, grid, block, 0, stream, C, P, splits,

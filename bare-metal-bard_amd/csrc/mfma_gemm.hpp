@@ -61,6 +61,9 @@ struct EpiArgs {
     const float *bias;  // EPI_BIAS*: N floats
     float *act;         // EPI_BIAS_GELU: M x N, same layout as C
     const float *pre;   // EPI_GELU_GRAD: the GELU input, M x N, same layout as C
+    // EPI_GELU_GRAD on the bf16x3 kernels only, or null: where wave tile row w
+    // writes the column sums of its rows of C, as row w of a (rows, N) array.
+    float *colsum;
 };
 
 // The fused epilogues are the reference's separate passes in one: gemm with

@@ -355,22 +355,27 @@ __global__ __launch_bounds__(NT) void ln_fwd_generic_k(float *out, float *mean, 
 //   dxhat = dout * w, xhat = (x - mean) * rstd.
 // The weight and bias gradients of the workgroup's rows are summed in
 // registers, combined across its waves through LDS in wave order, and written
-// as partial[blk][0:C] (dweight) and partial[blk][C:2C] (dbias).
+// as partial[blk][0:C] (dweight) and partial[blk][C:2C] (dbias). SUM: also the
+// column sums of the updated dinp, as partial[blk][2C:3C] (the gradient of a
+// bias whose layer's output dinp is the gradient of; its own pass over dinp
+// cost 5-10 us).
 constexpr int LN_WAVES = 8;
 
-template <int NCH, bool RAG>
+template <int NCH, bool RAG, bool SUM>
 __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
     float *dinp, float *partial, const float *dout, const float *inp, const float *weight,
     const float *mean, const float *rstd, int N, int C, int rpb) {
-    extern __shared__ float red[];  // [LN_WAVES][2C]
+    constexpr int OUT = SUM ? 3 : 2;
+    extern __shared__ float red[];  // [LN_WAVES][OUT * C]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float4 w[NCH], dw[NCH], db[NCH];
+    float4 w[NCH], dw[NCH], db[NCH], ds[SUM ? NCH : 1];
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
         w[k] = c < C ? ld_cols<RAG>(weight, c, C, 0.0f) : zero4();
         dw[k] = zero4();
         db[k] = zero4();
+        if (SUM) ds[k] = zero4();
     }
     const int r0 = blockIdx.x * rpb;
     const int r1 = min(N, r0 + rpb);
@@ -409,13 +414,16 @@ __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
                 o.z += rs * (g[k].z * w[k].z - m1 - xh[k].z * m2);
                 o.w += rs * (g[k].w * w[k].w - m1 - xh[k].w * m2);
                 st_cols<RAG>(dx, c, C, o);
+                if (SUM) {
+                    ds[k].x += o.x; ds[k].y += o.y; ds[k].z += o.z; ds[k].w += o.w;
+                }
                 dw[k].x += g[k].x * xh[k].x; dw[k].y += g[k].y * xh[k].y;
                 dw[k].z += g[k].z * xh[k].z; dw[k].w += g[k].w * xh[k].w;
                 db[k].x += g[k].x; db[k].y += g[k].y; db[k].z += g[k].z; db[k].w += g[k].w;
             }
         }
     }
-    float *mine = red + wave * 2 * C;
+    float *mine = red + wave * OUT * C;
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
         const int c = (k * 64 + lane) * 4;
@@ -423,18 +431,20 @@ __global__ __launch_bounds__(LN_WAVES * 64) void ln_bwd_k(
             if (RAG) {
                 st_cols<true>(mine, c, C, dw[k]);
                 st_cols<true>(mine + C, c, C, db[k]);
+                if (SUM) st_cols<true>(mine + 2 * C, c, C, ds[k]);
             } else {
                 bmb::st4(mine + c, dw[k]);
                 bmb::st4(mine + C + c, db[k]);
+                if (SUM) bmb::st4(mine + 2 * C + c, ds[k]);
             }
         }
     }
     __syncthreads();
-    for (int j = threadIdx.x; j < 2 * C; j += LN_WAVES * 64) {
+    for (int j = threadIdx.x; j < OUT * C; j += LN_WAVES * 64) {
         float s = red[j];
 #pragma unroll
-        for (int q = 1; q < LN_WAVES; ++q) s += red[q * 2 * C + j];
-        partial[(size_t)blockIdx.x * 2 * C + j] = s;
+        for (int q = 1; q < LN_WAVES; ++q) s += red[q * OUT * C + j];
+        partial[(size_t)blockIdx.x * OUT * C + j] = s;
     }
 }
 
@@ -518,32 +528,41 @@ __global__ __launch_bounds__(NT) void colsum4_k(float *partial, const float *dou
     reinterpret_cast<float4 *>(partial + (size_t)blockIdx.y * C)[c4] = s;
 }
 
-// dst0[c] += sum_g partial[g][c] for c < C0, dst1[c - C0] += ... for the rest
-// (width columns in all). A workgroup covers FIN_COLS columns with
+// Each job's column sums over its G partial rows, added onto its destinations
+// (ColsumJob). A workgroup covers FIN_COLS columns of one job with
 // NT / FIN_COLS slices of lanes: slice q sums g = q, q + slices, ... in order,
 // then the slice sums are added in slice order. Few columns per workgroup
 // and many slices keep each lane's chain of dependent adds short (the
 // partials are a few hundred rows and sit in L2; this kernel is latency-
-// bound, not bandwidth-bound).
+// bound, 4.8-5.2 us for one job, so a caller with several runs them at once).
 constexpr int FIN_COLS = 8;
-__global__ __launch_bounds__(NT) void colsum_finish_k(float *dst0, float *dst1, int C0,
-                                                       const float *partial, int G, int width) {
+struct ColsumJobs {
+    bmb::ColsumJob job[bmb::COLSUM_JOBS];
+    int first[bmb::COLSUM_JOBS + 1];  // job q: workgroups [first[q], first[q + 1])
+};
+__global__ __launch_bounds__(NT) void colsum_finish_k(ColsumJobs jobs) {
     constexpr int SL = NT / FIN_COLS;
     __shared__ float sl[SL][FIN_COLS];
-    const int col = threadIdx.x % FIN_COLS, q = threadIdx.x / FIN_COLS;
-    const int c = blockIdx.x * FIN_COLS + col;
+    int q = 0;
+    while (q + 1 < bmb::COLSUM_JOBS && (int)blockIdx.x >= jobs.first[q + 1]) ++q;
+    const bmb::ColsumJob &j = jobs.job[q];
+    const int width = j.n[0] + j.n[1] + j.n[2], G = j.G;
+    const int col = threadIdx.x % FIN_COLS, slice = threadIdx.x / FIN_COLS;
+    const int c = ((int)blockIdx.x - jobs.first[q]) * FIN_COLS + col;
     float s = 0.0f;
     if (c < width)
-        for (int g = q; g < G; g += SL) s += partial[(size_t)g * width + c];
-    sl[q][col] = s;
+        for (int g = slice; g < G; g += SL) s += j.partial[(size_t)g * width + c];
+    sl[slice][col] = s;
     __syncthreads();
-    if (q == 0 && c < width) {
+    if (slice == 0 && c < width) {
         float t = sl[0][col];
         for (int k = 1; k < SL; ++k) t += sl[k][col];
-        if (c < C0)
-            dst0[c] += t;
+        if (c < j.n[0])
+            j.dst[0][c] += t;
+        else if (c < j.n[0] + j.n[1])
+            j.dst[1][c - j.n[0]] += t;
         else
-            dst1[c - C0] += t;
+            j.dst[2][c - j.n[0] - j.n[1]] += t;
     }
 }
 
@@ -923,11 +942,6 @@ void colsum_shape(int N, int C, int &rpc, int &G) {
     G = ceil_div(N, rpc);
 }
 
-void colsum_finish(float *d0, float *d1, int C0, const float *partial, int G, int width) {
-    bmb::launch(colsum_finish_k, dim3(ceil_div(width, FIN_COLS)), dim3(NT), 0, nullptr, d0, d1,
-                C0, partial, G, width);
-}
-
 template <int NCH, bool RES>
 void ln_fwd_launch(float *out, float *mean, float *rstd, const float *inp, const float *w,
                    const float *b, int N, int C, float *res_out = nullptr,
@@ -953,15 +967,35 @@ bool ln_fwd_rows(float *out, float *mean, float *rstd, const float *inp, const f
     return true;
 }
 
-template <int NCH>
+// Row groups of the fused layernorm backward: G workgroups of rpb rows, about
+// 256 of them, whole waves of rows.
+void ln_bwd_shape(int N, int &rpb, int &G) {
+    const int G0 = std::max(1, std::min(256, ceil_div(N, LN_WAVES)));
+    rpb = ceil_div(ceil_div(N, G0), LN_WAVES) * LN_WAVES;
+    G = ceil_div(N, rpb);
+}
+
+template <int NCH, bool SUM>
 void ln_bwd_launch(float *dinp, float *partial, const float *dout, const float *inp,
                    const float *w, const float *mean, const float *rstd, int N, int C, int rpb,
                    int G) {
-    const size_t smem = (size_t)LN_WAVES * 2 * C * sizeof(float);
-    auto *kern = C % 4 == 0 ? ln_bwd_k<NCH, false> : ln_bwd_k<NCH, true>;
+    const size_t smem = (size_t)LN_WAVES * (SUM ? 3 : 2) * C * sizeof(float);
+    auto *kern = C % 4 == 0 ? ln_bwd_k<NCH, false, SUM> : ln_bwd_k<NCH, true, SUM>;
     bmb::allow_smem(kern, smem);
     bmb::launch(kern, dim3(G), dim3(LN_WAVES * 64), smem, nullptr, dinp, partial, dout, inp, w,
                 mean, rstd, N, C, rpb);
+}
+
+template <bool SUM>
+void ln_bwd_rows(float *dinp, float *partial, const float *dout, const float *inp, const float *w,
+                 const float *mean, const float *rstd, int N, int C, int rpb, int G) {
+    switch (row_chunks(C)) {
+        case 1: ln_bwd_launch<1, SUM>(dinp, partial, dout, inp, w, mean, rstd, N, C, rpb, G); break;
+        case 2: ln_bwd_launch<2, SUM>(dinp, partial, dout, inp, w, mean, rstd, N, C, rpb, G); break;
+        case 3: ln_bwd_launch<3, SUM>(dinp, partial, dout, inp, w, mean, rstd, N, C, rpb, G); break;
+        case 4: ln_bwd_launch<4, SUM>(dinp, partial, dout, inp, w, mean, rstd, N, C, rpb, G); break;
+        default: ln_bwd_launch<8, SUM>(dinp, partial, dout, inp, w, mean, rstd, N, C, rpb, G); break;
+    }
 }
 
 template <int NTHR, int NCH>
@@ -991,6 +1025,62 @@ void bmb::residual_layernorm_forward(float *res_out, float *ln_out, float *mean,
     if (ln_fwd_rows<true>(ln_out, mean, rstd, a, weight, bias, N, C, res_out, b)) return;
     residual_forward(res_out, a, b, N * C);
     layernorm_forward(ln_out, mean, rstd, res_out, weight, bias, N, C);
+}
+
+void bmb::colsum_finish_jobs(const ColsumJob *jobs, int count) {
+    if (count <= 0) return;
+    ColsumJobs a{};
+    for (int q = 0; q < COLSUM_JOBS; ++q) {
+        if (q < count) a.job[q] = jobs[q];
+        const int width = a.job[q].n[0] + a.job[q].n[1] + a.job[q].n[2];
+        a.first[q + 1] = a.first[q] + (q < count ? ceil_div(width, FIN_COLS) : 0);
+    }
+    launch(colsum_finish_k, dim3(a.first[COLSUM_JOBS]), dim3(NT), 0, nullptr, a);
+}
+
+size_t bmb::bias_partial_floats(int N, int C) {
+    int rpc, G;
+    colsum_shape(N, C, rpc, G);
+    return (size_t)G * C;
+}
+
+bmb::ColsumJob bmb::bias_backward_partial(float *dbias, const float *dout, int N, int C,
+                                          float *partial) {
+    int rpc, G;
+    colsum_shape(N, C, rpc, G);
+    if (C % 4 == 0 && ((uintptr_t)dout & 15u) == 0)
+        launch(colsum4_k, dim3(ceil_div(C / 4, NT), G), dim3(NT), 0, nullptr, partial, dout, N, C,
+               rpc);
+    else
+        launch(colsum_k<false>, dim3(ceil_div(C, NT), G), dim3(NT), 0, nullptr, partial, dout,
+               nullptr, nullptr, nullptr, N, C, rpc);
+    return ColsumJob{partial, {dbias, nullptr, nullptr}, {C, 0, 0}, G};
+}
+
+size_t bmb::layernorm_partial_floats(int N, int C) {
+    int rpb, G;
+    ln_bwd_shape(N, rpb, G);
+    return (size_t)G * 3 * C;
+}
+
+bool bmb::layernorm_backward_partial(float *dinp, float *dweight, float *dbias, float *dsum,
+                                     const float *dout, const float *inp, const float *weight,
+                                     const float *mean, const float *rstd, int N, int C,
+                                     float *partial, ColsumJob &job) {
+    // (The waves' sums of three columns arrays fit a CU's 160 KB of LDS.)
+    if (row_chunks(C) == 0 || (size_t)LN_WAVES * 3 * C * sizeof(float) > 160 * 1024) {
+        layernorm_backward(dinp, dweight, dbias, dout, inp, weight, mean, rstd, N, C);
+        if (dsum != nullptr) bias_backward(dsum, dinp, N, C);
+        return false;
+    }
+    int rpb, G;
+    ln_bwd_shape(N, rpb, G);
+    if (dsum != nullptr)
+        ln_bwd_rows<true>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G);
+    else
+        ln_bwd_rows<false>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G);
+    job = ColsumJob{partial, {dweight, dbias, dsum}, {C, C, dsum != nullptr ? C : 0}, G};
+    return true;
 }
 
 extern "C" {
@@ -1042,23 +1132,15 @@ void layernorm_backward(float *dinp, float *dweight, float *dbias, const float *
                         const float *inp, const float *weight, const float *mean,
                         const float *rstd, int N, int C) {
     if (N <= 0 || C <= 0) return;
-    const int nch = row_chunks(C);
-    if (nch > 0) {
-        // Workgroups of LN_WAVES waves, about 256 of them, whole waves of rows.
-        const int G0 = std::max(1, std::min(256, ceil_div(N, LN_WAVES)));
-        const int rpb = ceil_div(ceil_div(N, G0), LN_WAVES) * LN_WAVES;
-        const int G = ceil_div(N, rpb);
+    if (row_chunks(C) > 0) {
+        int rpb, G;
+        ln_bwd_shape(N, rpb, G);
         bmb::ScratchLease ws(bmb::SCRATCH_NN, (size_t)G * 2 * C * sizeof(float));
         if (!ws) scratch_failure("layernorm_backward");
         float *partial = static_cast<float *>(ws.get());
-        switch (nch) {
-            case 1: ln_bwd_launch<1>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
-            case 2: ln_bwd_launch<2>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
-            case 3: ln_bwd_launch<3>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
-            case 4: ln_bwd_launch<4>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
-            default: ln_bwd_launch<8>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G); break;
-        }
-        colsum_finish(dweight, dbias, C, partial, G, 2 * C);
+        ln_bwd_rows<false>(dinp, partial, dout, inp, weight, mean, rstd, N, C, rpb, G);
+        const bmb::ColsumJob job{partial, {dweight, dbias, nullptr}, {C, C, 0}, G};
+        bmb::colsum_finish_jobs(&job, 1);
         return;
     }
     int rpc, G;
@@ -1070,7 +1152,8 @@ void layernorm_backward(float *dinp, float *dweight, float *dbias, const float *
                 dout, inp, weight, mean, rstd, N, C);
     bmb::launch(colsum_k<true>, dim3(ceil_div(C, NT), G), dim3(NT), 0, nullptr, partial, dout,
                 inp, mean, rstd, N, C, rpc);
-    colsum_finish(dweight, dbias, C, partial, G, 2 * C);
+    const bmb::ColsumJob job{partial, {dweight, dbias, nullptr}, {C, C, 0}, G};
+    bmb::colsum_finish_jobs(&job, 1);
 }
 
 void gelu_forward(float *out, const float *inp, int n) { run_map(GeluFwd{out, inp}, n); }
@@ -1099,18 +1182,11 @@ void bias_forward(float *out, const float *bias, int N, int C) {
 
 void bias_backward(float *dbias, const float *dout, int N, int C) {
     if (N <= 0 || C <= 0) return;
-    int rpc, G;
-    colsum_shape(N, C, rpc, G);
-    bmb::ScratchLease ws(bmb::SCRATCH_NN, (size_t)G * C * sizeof(float));
+    bmb::ScratchLease ws(bmb::SCRATCH_NN, bmb::bias_partial_floats(N, C) * sizeof(float));
     if (!ws) scratch_failure("bias_backward");
-    float *partial = static_cast<float *>(ws.get());
-    if (C % 4 == 0 && ((uintptr_t)dout & 15u) == 0)
-        bmb::launch(colsum4_k, dim3(ceil_div(C / 4, NT), G), dim3(NT), 0, nullptr, partial, dout,
-                    N, C, rpc);
-    else
-        bmb::launch(colsum_k<false>, dim3(ceil_div(C, NT), G), dim3(NT), 0, nullptr, partial,
-                    dout, nullptr, nullptr, nullptr, N, C, rpc);
-    colsum_finish(dbias, dbias, C, partial, G, C);
+    const bmb::ColsumJob job =
+        bmb::bias_backward_partial(dbias, dout, N, C, static_cast<float *>(ws.get()));
+    bmb::colsum_finish_jobs(&job, 1);
 }
 
 void softmax_crossentropy_forward(float *probs, float *losses, const float *logits,

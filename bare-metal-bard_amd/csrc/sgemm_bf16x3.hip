@@ -640,6 +640,7 @@ struct Bf16x3Gemm {
         // is gathered before any result is stored: 16 * FN loads in flight.
         const int l32 = lane & 31, half = lane >> 5;
         const bool reads = (EPI == bmb::EPI_BLAS && beta != 0.0f) || EPI == bmb::EPI_GELU_GRAD;
+        float sums[FN] = {};  // of this lane's rows, per column (EPI_GELU_GRAD)
         float bias[FN];
         if (EPI == bmb::EPI_BIAS || EPI == bmb::EPI_BIAS_GELU) {
 #pragma unroll
@@ -679,13 +680,24 @@ struct Bf16x3Gemm {
                     } else if (EPI == bmb::EPI_BLAS) {
                         C[idx] = reads ? bmb::fma_rn(alpha, a, beta * in[fn][r]) : alpha * a;
                     } else if (EPI == bmb::EPI_GELU_GRAD) {
-                        C[idx] = bmb::gelu_grad(in[fn][r], a);
+                        const float v = bmb::gelu_grad(in[fn][r], a);
+                        C[idx] = v;
+                        sums[fn] += v;
                     } else {
                         const float v = a + bias[fn];
                         C[idx] = v;
                         if (EPI == bmb::EPI_BIAS_GELU) ep.act[idx] = bmb::gelu(v);
                     }
                 }
+            }
+        }
+        if (EPI == bmb::EPI_GELU_GRAD && ep.colsum != nullptr) {
+            const size_t w = (size_t)(m0 / BM) * Tl::WAVES_M + wave / Tl::WAVES_N;
+#pragma unroll
+            for (int fn = 0; fn < FN; ++fn) {
+                const int col = n0 + wn + fn * 32 + l32;
+                const float t = sums[fn] + __shfl_xor(sums[fn], 32, 64);
+                if (half == 0 && (INTERIOR || col < N)) ep.colsum[w * N + col] = t;
             }
         }
     }
@@ -1153,6 +1165,16 @@ void run_band(const Part &p, int M, int N, int K, float alpha, const float *A, c
     }
 }
 
+// Rows of partial column sums that a part of M rows writes (EpiArgs::colsum).
+int sum_rows(const Part &p, int M) {
+    if (p.tile == NARROW) return bmb::ceil_div(M, TileS::BM) * TileS::WAVES_M;
+    const int bm = CANDS[p.tile].bm;
+    return bmb::ceil_div(M, bm) * (bm == 32 ? TileXS::WAVES_M : TileS::WAVES_M);
+}
+static_assert(TileL::WAVES_M == TileS::WAVES_M && TileM::WAVES_M == TileS::WAVES_M &&
+                  TileT::WAVES_M == TileS::WAVES_M,
+              "sum_rows");
+
 // Both bands of a plan, in row order on one stream (the second band's split
 // partials reuse P after the first band's reduce has read it).
 template <bool TA, bool TB, int EPI>
@@ -1170,6 +1192,7 @@ void run_plan(const Plan &p, int M, int N, int K, float alpha, const float *A, c
     bmb::EpiArgs e1 = ep;
     if (e1.act) e1.act += r * N;
     if (e1.pre) e1.pre += r * N;
+    if (e1.colsum) e1.colsum += (size_t)sum_rows(p.part[0], p.m1) * N;
     // A band of rows starts r rows (TA: r columns of the stored K x M) in.
     const float *A1 = TA ? A + r : A + r * K;
     run_band<TA, TB, EPI>(p.part[1], M - p.m1, N, K, alpha, A1, B, beta, C + r * N, ld, P, stream,
@@ -1198,9 +1221,9 @@ long long partial_floats(const Plan &p, int M, int N, int K) {
 bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const float *A,
                       const float *B, float beta, float *C, hipStream_t stream, int epi,
                       const float *bias, float *act, const float *pre, float *fixed,
-                      long long fixed_floats) {
+                      long long fixed_floats, float *colsum, int *colsum_rows) {
     if (M <= 0 || N <= 0) return true;
-    const bmb::EpiArgs ep{bias, act, pre};
+    bmb::EpiArgs ep{bias, act, pre, nullptr};
     const bool may_split = fixed != nullptr || !bmb::stream_capturing(stream);
     const bool edges_ok = !ta && !tb && epi == bmb::EPI_BLAS;
     // (Every epilogue has k-sliced kernels, so a fused linear layer and
@@ -1218,6 +1241,11 @@ bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const 
         lease.emplace(bmb::SCRATCH_GEMM, (size_t)pf * sizeof(float), stream);
         P = static_cast<float *>(lease->get());
         if (P == nullptr) p = pick(M, N, K, mis_a, mis_b, false, 0, edges_ok, ks_ok);  // no scratch: no split
+    }
+    const bool banded = p.m1 < M;
+    if (colsum != nullptr && p.part[0].splits == 1 && (!banded || p.part[1].splits == 1)) {
+        ep.colsum = colsum;
+        *colsum_rows = sum_rows(p.part[0], p.m1) + (banded ? sum_rows(p.part[1], M - p.m1) : 0);
     }
 #define BMB_B3(TA_, TB_, EPI_)                                                              \
     run_plan<TA_, TB_, EPI_>(p, M, N, K, alpha, A, B, beta, C, P, stream, ep);              \

@@ -83,6 +83,28 @@ def test_forward_backward_vs_oracle(gpu, use_flash):
     print("logits %.2e, worst gradient %.2e" % (el, worst))
 
 
+# The backward's column sums come from the kernels that make the gradients:
+# rows that are no whole tile or wave of rows, a ragged width of the MLP, and a
+# width whose layernorm sums do not fit the fused kernel.
+@pytest.mark.parametrize("cfg,b", [((50, 65, 128, 2, 3, 96), 3), ((33, 65, 66, 1, 1, 32), 1),
+                                   ((8, 65, 128, 1, 16, 2048), 1)],
+                         ids=["C96", "C32", "C2048"])
+def test_gradients_at_other_widths(gpu, cfg, b):
+    n = b * cfg[0]
+    m = _model(True, cfg=cfg, b=b, t=cfg[0])
+    x, y = _batch(99, cfg[1], n)
+    print("gpt gradients", cfg, b, flush=True)
+    loss = m.forward(x, y)
+    m.backward()
+    sync("gpt backward")
+    ref_loss, _, ref_g, _ = O.gpt_forward_backward(cfg, b, cfg[0], _params(m), x, y)
+    assert abs(loss - ref_loss) <= 1e-5 * ref_loss
+    g, off = _grads(m), _offsets(cfg)
+    for t, name in enumerate(O.PARAM_NAMES):
+        e, bad = O.normwise(g[off[t]:off[t + 1]], ref_g[off[t]:off[t + 1]])
+        assert bad == 0 and e < 1e-4, (name, e)
+
+
 def _loss_double(m, x, y):
     """Mean loss with the per-position losses summed in fp64 on the host
     (tools/test_grad.cu:44-52)."""
