@@ -102,6 +102,7 @@ using TileL = B3Tile<256, 256, 2, 4>;
 using TileM = B3Tile<128, 128, 2, 2>;
 using TileS = B3Tile<64, 64, 2, 2>;
 using TileT = B3Tile<128, 256, 2, 4>;
+using TileH = B3Tile<128, 64, 2, 2>;  // k-sliced kernels only
 using TileXS = B3Tile<32, 32, 1, 1>;  // one wave (k-sliced kernels only)
 
 // Offset (in bf16) of element k (a multiple of 4) of LDS row `row`. Rows are
@@ -805,8 +806,8 @@ __global__ __launch_bounds__(TileS::NT) void bf16x3_narrow_k(int M, int N, int K
 
 // Tile and split choice. A work item is one output tile over one K range. A
 // CU that holds r items of a tile at once takes
-//   c + d r + stages (a + b r) (1 + mis u)
-// us for them: per 32-k stage a part that residents overlap (a, the latency
+//   c + d r + stages (a + b r) (1 + mis u) t
+// us for them (t: nt or tn by transposes, 1 for A B): per 32-k stage a part that residents overlap (a, the latency
 // chain of a stage) and one that they share (b, the CU's LDS, VALU and matrix
 // cores), a prologue c and an epilogue d. u is the share of the staged bytes
 // whose rows are not a multiple of 16 bytes apart. The device runs cus x
@@ -814,12 +815,12 @@ __global__ __launch_bounds__(TileS::NT) void bf16x3_narrow_k(int M, int N, int K
 // mean and its fullest CU. A split adds the partials' round trip, the reduce
 // launch and a term per range (each reduce lane adds its ranges one after
 // the other), every plan its launch and the write of C. The constants are a
-// least-squares fit (on log time) to 10,000 timed plans of 250 problems on
+// least-squares fit (on log time) to 13,000 timed plans of 331 problems on
 // one MI355X: every tile x slices x split below over the linear layers of
 // GPTs of width 256-1024 at 64-16384 rows in all three transposes, squares of
 // 192-4608 and random shapes (M, N, K of 64-8192, a third of them odd). On
 // those the model's plan is 1.8% slower than the best measured one on average
-// (5% at the 90th percentile); the model before it, fitted to the GPT-2
+// (6% at the 90th percentile); the model before it, fitted to the GPT-2
 // layers and squares alone, 3.1% (16%), and up to 1.9x on problems of few
 // tiles or short K.
 //
@@ -834,18 +835,20 @@ __global__ __launch_bounds__(TileS::NT) void bf16x3_narrow_k(int M, int N, int K
 struct B3Cand {
     int bm, bn, ks;  // tile, and k-slices per workgroup (bf16x3_ks_k)
     double a, b, c, d, mis;
+    double nt, tn;  // stages of A B^T and of A^T B (and A^T B^T) against A B
 };
 constexpr B3Cand CANDS[] = {
-    {256, 256, 1, 0.000, 2.196, 2.90, 2.87, 0.04},
-    {128, 128, 1, 0.253, 0.562, 2.05, 0.26, 0.08},
-    {64, 64, 1, 0.160, 0.213, 1.10, 0.04, 0.16},
-    {128, 256, 1, 0.000, 1.258, 1.93, 1.32, 0.04},
-    {64, 64, 2, 0.159, 0.437, 1.25, 0.00, 0.17},
-    {64, 64, 4, 0.321, 0.746, 0.59, 1.39, 0.24},
-    {32, 32, 4, 0.251, 0.322, 0.96, 0.00, 0.33},
-    {32, 32, 8, 0.317, 0.628, 0.56, 0.77, 0.38},
+    {256, 256, 1, 0.000, 2.316, 3.82, 1.02, 0.06, 0.95, 0.97},
+    {128, 128, 1, 0.251, 0.572, 2.07, 0.22, 0.11, 0.98, 1.04},
+    {64, 64, 1, 0.158, 0.234, 1.01, 0.04, 0.16, 0.89, 0.99},
+    {128, 256, 1, 0.019, 1.263, 1.19, 2.37, 0.08, 0.95, 1.02},
+    {64, 64, 2, 0.134, 0.498, 1.15, 0.00, 0.19, 0.89, 0.98},
+    {64, 64, 4, 0.118, 1.093, 0.76, 1.10, 0.20, 0.86, 0.95},
+    {32, 32, 4, 0.225, 0.331, 0.91, 0.00, 0.35, 0.94, 1.09},
+    {32, 32, 8, 0.300, 0.588, 0.14, 1.22, 0.42, 0.96, 1.11},
+    {128, 64, 2, 0.180, 0.785, 2.14, 0.00, 0.14, 0.94, 1.11},
 };
-constexpr int N_CANDS = 8;
+constexpr int N_CANDS = 9;
 constexpr int NARROW = N_CANDS;  // bf16x3_narrow_k, planned as the 64 x 64 tile
 // The 32 x 32 tile is only taken up to XS_MAX_OUTPUTS outputs, and every
 // slice keeps at least MIN_SLICE_K of k.
@@ -854,11 +857,11 @@ constexpr int MIN_SLICE_K = 64;
 // Split counts that are not powers of two fill the device in one round where
 // {2, 4, 8} do not (36 tiles of 256 x 256 in 7 ranges on 256 CUs).
 constexpr int SPLITS[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
-constexpr double LAUNCH_US = 3.3;                  // one launch, timed back to back
-constexpr double C_BYTES_PER_US = 15.5e6;          // the write of C
-constexpr double PARTIALS_BYTES_PER_US = 11.9e6;   // the partials' round trip
-constexpr double REDUCE_US = 1.1, RANGE_US = 0.27;  // the reduce, and each range in it
-constexpr double FULLEST = 0.67;  // a partial round: the weight of its fullest CU
+constexpr double LAUNCH_US = 3.5;                 // one launch, timed back to back
+constexpr double C_BYTES_PER_US = 13.0e6;         // the write of C
+constexpr double PARTIALS_BYTES_PER_US = 11.0e6;  // the partials' round trip
+constexpr double REDUCE_US = 1.1, RANGE_US = 0.24;  // the reduce, and each range in it
+constexpr double FULLEST = 0.65;  // a partial round: the weight of its fullest CU
 // A second band: its launch and the drain between the bands. Bands are only
 // tried for K >= MIN_BAND_K, with K ranges of at least MIN_BAND_SPLIT_K in a
 // split remainder band, and taken when modelled 3% faster than one band:
@@ -933,6 +936,7 @@ const Device &device_info(int dev) {
         d.occ[5] = ks_occupancy_of<TileS, 4>();
         d.occ[6] = ks_occupancy_of<TileXS, 4>();
         d.occ[7] = ks_occupancy_of<TileXS, 8>();
+        d.occ[8] = ks_occupancy_of<TileH, 2>();
         int c = 0;
         if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             c <= 0) {
@@ -944,11 +948,17 @@ const Device &device_info(int dev) {
     return info[dev];
 }
 
+// What a plan depends on besides M, N and K: the transposes, and whether an
+// operand's rows are not 16-byte aligned.
+struct Layout {
+    bool ta, tb, mis_a, mis_b;
+};
+
 // Modelled time (us) of an M x N x K band on tile t with K split s ways;
 // false if that split is not allowed (may_split, max_floats caps splits * M *
-// N). mis_a, mis_b: the operand's rows are not 16-byte aligned.
-bool part_time(const Device &dv, int M, int N, int K, int t, int s, bool mis_a, bool mis_b,
-               bool may_split, long long max_floats, Part &out, double &time) {
+// N).
+bool part_time(const Device &dv, int M, int N, int K, int t, int s, Layout lo, bool may_split,
+               long long max_floats, Part &out, double &time) {
     const B3Cand &c = CANDS[t];
     // The staging loads' byte offsets within a tile stay below 2^32.
     if (std::max(c.bm, c.bn) * (long long)K >= 1LL << 30 ||
@@ -974,8 +984,9 @@ bool part_time(const Device &dv, int M, int N, int K, int t, int s, bool mis_a, 
     const int occ = dv.occ[t], cus = dv.cus;
     const double stages = bmb::ceil_div(bmb::ceil_div(kchunk, BK), c.ks);
     const double share = (double)c.bm / (c.bm + c.bn);  // of the staged bytes, A's
-    const double mis = 1.0 + c.mis * ((mis_a ? share : 0.0) + (mis_b ? 1.0 - share : 0.0));
-    auto round = [&](double r) { return c.c + c.d * r + stages * (c.a + c.b * r) * mis; };
+    const double mis = 1.0 + c.mis * ((lo.mis_a ? share : 0.0) + (lo.mis_b ? 1.0 - share : 0.0));
+    const double rate = mis * (lo.ta ? c.tn : lo.tb ? c.nt : 1.0);
+    auto round = [&](double r) { return c.c + c.d * r + stages * (c.a + c.b * r) * rate; };
     const long long slots = (long long)cus * occ, rem = items % slots;
     time = (items / slots) * round(occ) + LAUNCH_US + mn * 4.0 / C_BYTES_PER_US;
     if (rem)
@@ -990,7 +1001,7 @@ bool part_time(const Device &dv, int M, int N, int K, int t, int s, bool mis_a, 
 
 // The fastest single-band plan of an M x N x K band (split K ranges of at
 // least min_split_k; k-sliced tiles only if ks_ok).
-double best_part(const Device &dv, int M, int N, int K, bool mis_a, bool mis_b, bool may_split,
+double best_part(const Device &dv, int M, int N, int K, Layout lo, bool may_split,
                  long long max_floats, Part &best, int min_split_k = 0, bool ks_ok = false) {
     double best_t = -1.0;
     const bool narrow = std::min({M, N, K}) < MIN_DIM;
@@ -1000,7 +1011,7 @@ double best_part(const Device &dv, int M, int N, int K, bool mis_a, bool mis_b, 
             if ((CANDS[t].ks > 1 && !ks_ok) || (narrow && t != 2)) continue;
             Part p;
             double tm;
-            if (part_time(dv, M, N, K, t, s, mis_a, mis_b, may_split, max_floats, p, tm) &&
+            if (part_time(dv, M, N, K, t, s, lo, may_split, max_floats, p, tm) &&
                 (p.splits == 1 || p.kchunk >= min_split_k) && (best_t < 0 || tm < best_t)) {
                 best_t = tm;
                 best = p;
@@ -1012,12 +1023,12 @@ double best_part(const Device &dv, int M, int N, int K, bool mis_a, bool mis_b, 
 }
 
 // ks_ok: the k-sliced tiles may run the problem (single-band plans only).
-Plan plan_for(int dev, int M, int N, int K, bool mis_a, bool mis_b, bool may_split,
-              long long max_floats, bool edges_ok, bool ks_ok) {
+Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long max_floats,
+              bool edges_ok, bool ks_ok) {
     const Device &dv = device_info(dev);
     Plan best{{Part{0, 1, K}, Part{0, 1, K}}, M, N, false};
     const double single_t =
-        best_part(dv, M, N, K, mis_a, mis_b, may_split, max_floats, best.part[0], 0, ks_ok);
+        best_part(dv, M, N, K, lo, may_split, max_floats, best.part[0], 0, ks_ok);
     double best_t = single_t;
     // Two bands: the first whole rounds of one tile, the rest on its own plan.
     for (int t = 0; K >= MIN_BAND_K && std::min(M, N) >= MIN_DIM && t < N_CANDS; ++t) {
@@ -1033,8 +1044,8 @@ Plan plan_for(int dev, int M, int N, int K, bool mis_a, bool mis_b, bool may_spl
             if (M - m1 < MIN_DIM) continue;
             Part p0, p1;
             double t0, t1;
-            if (!part_time(dv, m1, N, K, t, 1, mis_a, mis_b, false, 0, p0, t0)) continue;
-            t1 = best_part(dv, M - m1, N, K, mis_a, mis_b, may_split, max_floats, p1,
+            if (!part_time(dv, m1, N, K, t, 1, lo, false, 0, p0, t0)) continue;
+            t1 = best_part(dv, M - m1, N, K, lo, may_split, max_floats, p1,
                            MIN_BAND_SPLIT_K);
             const double tm = t0 + t1 + BAND_US;
             if (tm < BAND_GAIN * single_t && tm < best_t) {
@@ -1055,7 +1066,7 @@ Plan plan_for(int dev, int M, int N, int K, bool mis_a, bool mis_b, bool may_spl
             continue;
         Part p0;
         double t0;
-        if (!part_time(dv, m1, n1, K, t, 1, mis_a, mis_b, false, 0, p0, t0)) continue;
+        if (!part_time(dv, m1, n1, K, t, 1, lo, false, 0, p0, t0)) continue;
         const double tm = t0 + 1e6 * bmb::edge_model_s(m1, N - n1, M - m1, N, K);
         if (tm < BAND_GAIN * single_t && tm < best_t) {
             best_t = tm;
@@ -1071,26 +1082,51 @@ Plan plan_for(int dev, int M, int N, int K, bool mis_a, bool mis_b, bool may_spl
     return best;
 }
 
-// Plans are memoised per (device, shape, split permission and cap): the
-// search above costs tens of microseconds, a GEMM call in a training step
-// a few hundred.
-Plan pick(int M, int N, int K, bool mis_a, bool mis_b, bool may_split, long long max_floats,
-          bool edges_ok, bool ks_ok) {
+// Plans are memoised per (device, shape, layout, split permission and cap):
+// the search above costs tens of microseconds, a GEMM call in a training step
+// a few hundred. Each host thread keeps its last plans in a table of its own
+// in front of the shared map, so that a repeated call neither locks nor walks
+// the map.
+struct PlanKey {
+    int dev, M, N, K;
+    Layout lo;
+    bool may_split, edges_ok, ks_ok;
+    long long max_floats;
+    auto tie() const { return std::tie(dev, M, N, K, lo.ta, lo.tb, lo.mis_a, lo.mis_b, may_split,
+                                       edges_ok, ks_ok, max_floats); }
+    bool operator<(const PlanKey &o) const { return tie() < o.tie(); }
+    bool operator==(const PlanKey &o) const { return tie() == o.tie(); }
+};
+
+Plan pick(int M, int N, int K, Layout lo, bool may_split, long long max_floats, bool edges_ok,
+          bool ks_ok) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    using Key = std::tuple<int, int, int, int, bool, bool, bool, long long, bool, bool>;
+    const PlanKey key{dev, M, N, K, lo, may_split, edges_ok, ks_ok, max_floats};
+    struct Entry {
+        PlanKey key;
+        Plan plan;
+    };
+    static thread_local Entry recent[64] = {};  // (M = 0 is never planned)
+    const unsigned h = ((unsigned)M * 2654435761u) ^ ((unsigned)N * 40503u) ^ (unsigned)K * 97u ^
+                       (lo.ta ? 5u : 0u) ^ (lo.tb ? 10u : 0u);
+    Entry &e = recent[(h ^ (h >> 13)) % 64];
+    if (e.key == key) return e.plan;
     static std::mutex mu;
-    static std::map<Key, Plan> memo;
-    const Key key{dev, M, N, K, mis_a, mis_b, may_split, max_floats, edges_ok, ks_ok};
+    static std::map<PlanKey, Plan> memo;
     {
         std::lock_guard<std::mutex> lock(mu);
-        auto it = memo.find(key);
-        if (it != memo.end()) return it->second;
+        const auto it = memo.find(key);
+        if (it != memo.end()) {
+            e = Entry{key, it->second};
+            return e.plan;
+        }
     }
-    const Plan p = plan_for(dev, M, N, K, mis_a, mis_b, may_split, max_floats, edges_ok, ks_ok);
+    const Plan p = plan_for(dev, M, N, K, lo, may_split, max_floats, edges_ok, ks_ok);
     std::lock_guard<std::mutex> lock(mu);
     if (memo.size() > 4096) memo.clear();
     memo.emplace(key, p);
+    e = Entry{key, p};
     return p;
 }
 
@@ -1141,6 +1177,7 @@ void launch_tile(int M, int N, int K, const Part &p, float alpha, const float *A
     case 5: launch_ks<TileS, TA, TB, EPI, 4>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
     case 6: launch_ks<TileXS, TA, TB, EPI, 4>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
     case 7: launch_ks<TileXS, TA, TB, EPI, 8>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
+    case 8: launch_ks<TileH, TA, TB, EPI, 2>(M, N, K, p, alpha, A, B, beta, C, ld, stream, ep); break;
     default:
         bmb::launch(bf16x3_narrow_k<TA, TB, EPI>,
                     dim3(bmb::ceil_div(M, TileS::BM) * bmb::ceil_div(N, TileS::BN), p.splits),
@@ -1172,7 +1209,7 @@ int sum_rows(const Part &p, int M) {
     return bmb::ceil_div(M, bm) * (bm == 32 ? TileXS::WAVES_M : TileS::WAVES_M);
 }
 static_assert(TileL::WAVES_M == TileS::WAVES_M && TileM::WAVES_M == TileS::WAVES_M &&
-                  TileT::WAVES_M == TileS::WAVES_M,
+                  TileT::WAVES_M == TileS::WAVES_M && TileH::WAVES_M == TileS::WAVES_M,
               "sum_rows");
 
 // Both bands of a plan, in row order on one stream (the second band's split
@@ -1230,9 +1267,9 @@ bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const 
     // gemm() plus the separate bias/GELU pass plan a shape alike and give the
     // same bits.)
     const bool ks_ok = true;
-    const bool mis_a = (ta ? M : K) % 4 != 0 || ((uintptr_t)A & 15) != 0;
-    const bool mis_b = (tb ? K : N) % 4 != 0 || ((uintptr_t)B & 15) != 0;
-    Plan p = pick(M, N, K, mis_a, mis_b, may_split, fixed ? fixed_floats : MAX_SPLIT_FLOATS,
+    const Layout lo{ta, tb, (ta ? M : K) % 4 != 0 || ((uintptr_t)A & 15) != 0,
+                    (tb ? K : N) % 4 != 0 || ((uintptr_t)B & 15) != 0};
+    Plan p = pick(M, N, K, lo, may_split, fixed ? fixed_floats : MAX_SPLIT_FLOATS,
                   edges_ok, ks_ok);
     float *P = fixed;
     std::optional<bmb::ScratchLease> lease;
@@ -1240,7 +1277,7 @@ bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const 
     if (pf > 0 && fixed == nullptr) {
         lease.emplace(bmb::SCRATCH_GEMM, (size_t)pf * sizeof(float), stream);
         P = static_cast<float *>(lease->get());
-        if (P == nullptr) p = pick(M, N, K, mis_a, mis_b, false, 0, edges_ok, ks_ok);  // no scratch: no split
+        if (P == nullptr) p = pick(M, N, K, lo, false, 0, edges_ok, ks_ok);  // no scratch: no split
     }
     const bool banded = p.m1 < M;
     if (colsum != nullptr && p.part[0].splits == 1 && (!banded || p.part[1].splits == 1)) {
