@@ -216,8 +216,11 @@ def sgemm(kid: int, M, N, K, alpha, A, B, beta, C) -> None:
 
 
 # ------------------------------------------------------------ gemm.h
+# (The calls that a training or sampling loop makes hundreds of times a step
+# do as little here as they can: a short GEMM takes the GPU no longer than
+# Python takes to queue it.)
 def gemm(ta, tb, M, N, K, alpha, A, B, beta, C, stream=0) -> None:
-    lib().gemm(bool(ta), bool(tb), M, N, K, alpha, A, B, beta, C, stream or None)
+    (_lib or lib()).gemm(ta, tb, M, N, K, alpha, A, B, beta, C, stream or None)
 
 
 GEMM_MATH_BF16X3, GEMM_MATH_FP32 = 0, 1  # include/gemm.h
@@ -225,7 +228,7 @@ GEMM_MATH_BF16X3, GEMM_MATH_FP32 = 0, 1  # include/gemm.h
 
 def gemm_set_math(math: int) -> int:
     """Selects gemm()'s arithmetic for the process; returns the previous mode."""
-    return int(lib().gemm_set_math(int(math)))
+    return (_lib or lib()).gemm_set_math(int(math))
 
 
 def gemm_get_math() -> int:
@@ -235,18 +238,19 @@ def gemm_get_math() -> int:
 class gemm_math:
     """`with bmb.gemm_math(bmb.GEMM_MATH_FP32): ...` runs the block in that
     mode and restores the previous one."""
+    __slots__ = ("math", "prev")
 
     def __init__(self, math):
         self.math, self.prev = math, None
 
     def __enter__(self):
-        self.prev = gemm_set_math(self.math)
+        self.prev = (_lib or lib()).gemm_set_math(int(self.math))
         if self.prev < 0:
             raise ValueError("unknown gemm math mode %r" % (self.math,))
         return self
 
     def __exit__(self, *exc):
-        gemm_set_math(self.prev)
+        _lib.gemm_set_math(self.prev)
         return False
 
 
@@ -296,7 +300,7 @@ def flash_default_bwd_config() -> int:
 def call(name, *args):
     """Calls the C entry point `name` with raw arguments (device pointers as
     ints); returns its result."""
-    return getattr(lib(), name)(*args)
+    return getattr(_lib or lib(), name)(*args)
 
 
 def param_names():
