@@ -734,8 +734,8 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *pr
 // ------------------------------------------------------- softmax + cross-entropy
 // One workgroup of NTHR lanes per row, the row's first V logits held in NCH
 // float4 registers per lane (V <= 4*NTHR*NCH; RAG: Vp % 4 != 0, chunks placed
-// as in xent_bwd_k and V <= 4*NTHR*NCH - 3; 2048 x 50257 498 -> 263 us against
-// the three-pass kernel below): max, then
+// as in xent_bwd_k and V <= 4*NTHR*NCH - 3; 2048 x 50257 485 -> 233 us against
+// the three-pass kernel below, 498 -> 263 traced): max, then
 // exp(x - max) and its sum, then the normalised probabilities -- one read of
 // the logits and one write of the probabilities (src/nn.cu:197-221).
 // exp(x - m) is exp2((x - m) * log2 e) on v_exp_f32.

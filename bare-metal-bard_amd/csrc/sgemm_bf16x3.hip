@@ -18,7 +18,8 @@
 //
 // Tiles. 256x256 (8 waves of 128x64), 128x256 (8 waves of 64x64), 128x128
 // (4 waves of 64x64) and 64x64 (4 waves of 32x32) outputs, K in stages of 32
-// (two 16-k MFMA steps), and a
+// (two 16-k MFMA steps); for few tiles, workgroups whose wave groups each take
+// every S-th stage (bf16x3_ks_k: 128x64, 64x64 and 32x32 outputs); and a
 // split of K into ranges whose fp32 partials one reduce adds in range order
 // (deterministic). A planner picks tile and split per shape, as gemm() does
 // for the fp32 MFMA path: the 256x256 tile alone leaves most CUs idle below
