@@ -734,8 +734,8 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *pr
 // ------------------------------------------------------- softmax + cross-entropy
 // One workgroup of NTHR lanes per row, the row's first V logits held in NCH
 // float4 registers per lane (V <= 4*NTHR*NCH; RAG: Vp % 4 != 0, chunks placed
-// as in xent_bwd_k and V <= 4*NTHR*NCH - 3; 2048 x 50257 485 -> 233 us against
-// the three-pass kernel below, 498 -> 263 traced): max, then
+// as in xent_bwd_k and V <= 4*NTHR*NCH - 3; 2048 x 50257 485 -> 222 us against
+// the three-pass kernel below): max, then
 // exp(x - max) and its sum, then the normalised probabilities -- one read of
 // the logits and one write of the probabilities (src/nn.cu:197-221).
 // exp(x - m) is exp2((x - m) * log2 e) on v_exp_f32.
@@ -811,7 +811,8 @@ __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *loss
     for (int k = 0; k < NCH; ++k) {
         const int c = first + (k * NTHR + tid) * 4;
         const float4 o = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
-        if (RAG ? c >= 0 && c + 3 < Vp : c < Vp) STREAM ? stu4_nt(p + c, o) : stu4(p + c, o);  // columns in [V, Vp) come out as exp2(-inf) = 0
+        // (Columns in [V, Vp) come out as exp2(-inf) = 0.)
+        if (RAG ? c >= 0 && c + 3 < Vp : c < Vp) STREAM ? stu4_nt(p + c, o) : stu4(p + c, o);
         if (tgt >= c && tgt < c + 4 && tgt >= 0 && tgt < V) {
             const int j = tgt - c;
             const float pt = j == 0 ? o.x : j == 1 ? o.y : j == 2 ? o.z : o.w;
@@ -820,6 +821,12 @@ __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *loss
     }
     for (int c = first + (NCH * NTHR + tid) * 4; c < Vp; c += NTHR * 4)
         if (!RAG || c + 3 < Vp) stu4(p + c, zero4());
+    // A row with a NaN or an infinity (uniform, rare): 0 * inv made its padding
+    // NaN; each lane clears what it wrote there. (Zeroed before the store, every
+    // row paid for it: 0.8 us of 10 at 64 x 50304.)
+    if (!(inv < INFINITY))
+        for (int c = first + tid * 4; c < Vp; c += NTHR * 4)
+            for (int j = max(c, V); j < min(c + 4, Vp); ++j) p[j] = 0.0f;
     if (RAG) {
         // The columns of the row's partial chunks (up to three at each end),
         // one lane each, from the logits again (with the same arithmetic).

@@ -222,6 +222,35 @@ def test_softmax_crossentropy(gpu, N, V, Vp):
     assert np.array_equal(dl.get().reshape(N, Vp), want)
 
 
+# A row that holds a NaN or an infinity has no distribution (all its
+# probabilities may be NaN), but its padding columns are zeros like any other
+# row's, and its neighbours are not touched. Widths on each kernel, aligned and
+# ragged, with padding inside the last chunk that holds a logit and beyond it.
+@pytest.mark.parametrize("V,Vp", [(65, 66), (65, 71), (63, 64), (1021, 1023), (1000, 1003),
+                                  (4095, 4099), (50257, 50263), (50257, 50304), (70000, 70003)])
+def test_softmax_padding_is_zero_in_rows_without_a_distribution(gpu, V, Vp):
+    N = 6
+    logits = _f32(_rng(17).standard_normal((N, Vp)) * 3)
+    logits[1, V // 2] = np.inf
+    logits[2, :] = -np.inf
+    logits[4, V - 1] = np.nan
+    tg = np.arange(N, dtype=np.int32) % V
+    print("softmax padding V=%d Vp=%d" % (V, Vp), flush=True)
+    probs, losses = Guarded(N * Vp, poison=True), Guarded(N, poison=True)
+    d_logits, d_tg = dev(logits), _itok(tg)
+    bmb.call("softmax_crossentropy_forward", probs.ptr, losses.ptr, d_logits.data_ptr(),
+             d_tg.data_ptr(), N, V, Vp)
+    sync("softmax_crossentropy_forward")
+    assert probs.ok() and losses.ok()
+    p = probs.get().reshape(N, Vp)
+    assert np.all(p[:, V:] == 0.0)
+    good = [0, 3, 5]
+    rp, rl = O.softmax_xent_fwd(logits[good], tg[good], len(good), V, Vp)
+    assert _nw(p[good], rp) < TOL
+    assert np.abs(losses.get()[good] - rl).max() < TOL * max(1.0, np.abs(rl).max())
+    assert np.isnan(p[[1, 2, 4], :V]).any(axis=1).all()
+
+
 def test_softmax_crossentropy_bad_targets_give_nan(gpu):
     N, V, Vp = 4, 10, 12
     logits = _f32(_rng(7).standard_normal((N, Vp)))
