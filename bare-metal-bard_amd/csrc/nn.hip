@@ -1005,6 +1005,14 @@ void ln_bwd_rows(float *dinp, float *partial, const float *dout, const float *in
     }
 }
 
+// One workgroup of nt lanes per row, N rows in as many launches as that takes:
+// a dispatch holds fewer than 2^32 lanes. go(r, n): rows [r, r + n).
+template <class F>
+void rows_in_launches(int N, int nt, F &&go) {
+    const int most = (int)(((1LL << 32) - 1) / nt);
+    for (int r = 0; r < N; r += std::min(most, N - r)) go(r, std::min(most, N - r));
+}
+
 template <int NTHR, int NCH>
 void xent_launch(float *probs, float *losses, const float *logits, const int *targets, int N,
                  int V, int Vp) {
@@ -1013,7 +1021,11 @@ void xent_launch(float *probs, float *losses, const float *logits, const int *ta
                                        : softmax_xent_k<NTHR, NCH, false, false>)
                              : (stream ? softmax_xent_k<NTHR, NCH, true, true>
                                        : softmax_xent_k<NTHR, NCH, true, false>);
-    bmb::launch(kern, dim3(N), dim3(NTHR), 0, nullptr, probs, losses, logits, targets, V, Vp);
+    rows_in_launches(N, NTHR, [&](int r, int n) {
+        const size_t off = (size_t)r * Vp;
+        bmb::launch(kern, dim3(n), dim3(NTHR), 0, nullptr, probs + off, losses + r, logits + off,
+                    targets + r, V, Vp);
+    });
 }
 
 float scalar_result(const float *dptr) {
@@ -1207,8 +1219,11 @@ void softmax_crossentropy_forward(float *probs, float *losses, const float *logi
         if (span <= 32768) return xent_launch<1024, 8>(probs, losses, logits, targets, N, V, Vp);
         if (span <= 65536) return xent_launch<1024, 16>(probs, losses, logits, targets, N, V, Vp);
     }
-    bmb::launch(softmax_xent_generic_k, dim3(N), dim3(NT), 0, nullptr, probs, losses, logits,
-                targets, V, Vp);
+    rows_in_launches(N, NT, [&](int r, int n) {
+        const size_t off = (size_t)r * Vp;
+        bmb::launch(softmax_xent_generic_k, dim3(n), dim3(NT), 0, nullptr, probs + off, losses + r,
+                    logits + off, targets + r, V, Vp);
+    });
 }
 
 void crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets,

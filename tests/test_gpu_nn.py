@@ -251,6 +251,36 @@ def test_softmax_padding_is_zero_in_rows_without_a_distribution(gpu, V, Vp):
     assert np.isnan(p[[1, 2, 4], :V]).any(axis=1).all()
 
 
+def test_softmax_more_rows_than_one_launch_holds(gpu):
+    """Rows of 4097 take 1024-lane workgroups, of which a dispatch holds fewer
+    than 2^22: the rows beyond run in a second launch. (In place, so that one
+    69 GB buffer is enough; rows of equal logits but for a few.)"""
+    V = Vp = 4097
+    N = (1 << 22) + 5
+    rows = [0, 1, (1 << 22) - 2, (1 << 22) - 1, 1 << 22, (1 << 22) + 3, N - 1]
+    logits = _f32(_rng(18).standard_normal((len(rows), Vp)) * 3)
+    tg = (np.arange(N) % V).astype(np.int32)
+    print("softmax rows N=%d V=%d" % (N, V), flush=True)
+    x = torch.zeros(N * Vp, dtype=torch.float32, device="cuda")
+    for i, r in enumerate(rows):
+        x[r * Vp:(r + 1) * Vp] = dev(logits[i])
+    losses, d_tg = Guarded(N, poison=True), _itok(tg)
+    bmb.call("softmax_crossentropy_forward", x.data_ptr(), losses.ptr, x.data_ptr(),
+             d_tg.data_ptr(), N, V, Vp)
+    sync("softmax_crossentropy_forward")
+    assert losses.ok()
+    rp, rl = O.softmax_xent_fwd(logits, tg[rows], len(rows), V, Vp)
+    got = np.stack([x[r * Vp:(r + 1) * Vp].cpu().numpy() for r in rows])
+    del x
+    torch.cuda.empty_cache()
+    assert _nw(got, rp) < TOL
+    l = losses.get()
+    assert np.abs(l[rows] - rl).max() < TOL * np.abs(rl).max()
+    same = np.ones(N, bool)
+    same[rows] = False
+    assert np.abs(l[same] - np.log(V)).max() < TOL * np.log(V)
+
+
 def test_softmax_crossentropy_bad_targets_give_nan(gpu):
     N, V, Vp = 4, 10, 12
     logits = _f32(_rng(7).standard_normal((N, Vp)))
