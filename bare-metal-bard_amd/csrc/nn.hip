@@ -71,28 +71,29 @@ inline unsigned grid_for(long long items) {
     return (unsigned)((items + NT - 1) / NT);
 }
 
-// Columns c..c+3 of a row of C: whole, or (RAG) those of them that exist, the
-// others as `fill`.
+// Columns c..c+3 (c >= -3) of a row of C: whole, or (RAG) those of them that
+// exist, the others as `fill`. (c + 3 may pass the largest int: c is compared
+// with C - 3.)
 template <bool RAG>
 __device__ __forceinline__ float4 ld_cols(const float *row, int c, int C, float fill) {
-    if (!RAG || (c >= 0 && c + 3 < C)) return ldu4(row + c);
+    if (!RAG || (c >= 0 && c < C - 3)) return ldu4(row + c);
     float4 v = make_float4(fill, fill, fill, fill);
-    if (c + 0 >= 0 && c + 0 < C) v.x = row[c + 0];
-    if (c + 1 >= 0 && c + 1 < C) v.y = row[c + 1];
-    if (c + 2 >= 0 && c + 2 < C) v.z = row[c + 2];
-    if (c + 3 >= 0 && c + 3 < C) v.w = row[c + 3];
+    if (c >= 0 && c < C) v.x = row[c];
+    if (c >= -1 && c < C - 1) v.y = row[c + 1];
+    if (c >= -2 && c < C - 2) v.z = row[c + 2];
+    if (c >= -3 && c < C - 3) v.w = row[c + 3];
     return v;
 }
 template <bool RAG>
 __device__ __forceinline__ void st_cols(float *row, int c, int C, float4 v) {
-    if (!RAG || (c >= 0 && c + 3 < C)) {
+    if (!RAG || (c >= 0 && c < C - 3)) {
         stu4(row + c, v);
         return;
     }
-    if (c + 0 >= 0 && c + 0 < C) row[c + 0] = v.x;
-    if (c + 1 >= 0 && c + 1 < C) row[c + 1] = v.y;
-    if (c + 2 >= 0 && c + 2 < C) row[c + 2] = v.z;
-    if (c + 3 >= 0 && c + 3 < C) row[c + 3] = v.w;
+    if (c >= 0 && c < C) row[c] = v.x;
+    if (c >= -1 && c < C - 1) row[c + 1] = v.y;
+    if (c >= -2 && c < C - 2) row[c + 2] = v.z;
+    if (c >= -3 && c < C - 3) row[c + 3] = v.w;
 }
 
 // ------------------------------------------------------------ row/column maps
@@ -715,15 +716,17 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *pr
     const float *p = probs + (size_t)r * Vp;
     float *d = dlogits + (size_t)r * Vp;
     const int first = RAG ? -(int)(((size_t)r * Vp) & 3) : 0;
-    const int c = first + (part * NT + (int)threadIdx.x) * 4;
-    if (c >= Vp) return;
+    const unsigned c3 = (part * NT + threadIdx.x) * 4 + (first + 3);  // c + 3, as unsigned
+    if (c3 >= Vp + 3u) return;
+    const int c = (int)(c3 - 3);
     const float4 v = ld_cols<RAG>(p, c, Vp, 0.0f);
+    const unsigned hit = (unsigned)tgt - (unsigned)c;  // the target's place in the chunk
     float4 o;
-    o.x = c + 0 < V ? (v.x - (c + 0 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-    o.y = c + 1 < V ? (v.y - (c + 1 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-    o.z = c + 2 < V ? (v.z - (c + 2 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-    o.w = c + 3 < V ? (v.w - (c + 3 == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
-    if (RAG && (c < 0 || c + 3 >= Vp))
+    o.x = c < V - 0 ? (v.x - (hit == 0 ? 1.0f : 0.0f)) * scale : 0.0f;
+    o.y = c < V - 1 ? (v.y - (hit == 1 ? 1.0f : 0.0f)) * scale : 0.0f;
+    o.z = c < V - 2 ? (v.z - (hit == 2 ? 1.0f : 0.0f)) * scale : 0.0f;
+    o.w = c < V - 3 ? (v.w - (hit == 3 ? 1.0f : 0.0f)) * scale : 0.0f;
+    if (RAG && (c < 0 || c >= Vp - 3))
         st_cols<true>(d, c, Vp, o);
     else if (nt)
         stu4_nt(d + c, o);
@@ -819,21 +822,22 @@ __global__ __launch_bounds__(NTHR) void softmax_xent_k(float *probs, float *loss
             losses[row] = xent_loss(pt);
         }
     }
-    for (int c = first + (NCH * NTHR + tid) * 4; c < Vp; c += NTHR * 4)
-        if (!RAG || c + 3 < Vp) stu4(p + c, zero4());
+    // (Unsigned: c passes the largest int behind a Vp near it.)
+    for (unsigned c = first + (NCH * NTHR + tid) * 4; c < (unsigned)Vp; c += NTHR * 4)
+        if (!RAG || (int)c < Vp - 3) stu4(p + c, zero4());
     // A row with a NaN or an infinity (uniform, rare): 0 * inv made its padding
     // NaN; each lane clears what it wrote there. (Zeroed before the store, every
     // row paid for it: 0.8 us of 10 at 64 x 50304.)
     if (!(inv < INFINITY))
-        for (int c = first + tid * 4; c < Vp; c += NTHR * 4)
+        for (int c = first + tid * 4; c < min(Vp, NCH * NTHR * 4); c += NTHR * 4)
             for (int j = max(c, V); j < min(c + 4, Vp); ++j) p[j] = 0.0f;
     if (RAG) {
         // The columns of the row's partial chunks (up to three at each end),
         // one lane each, from the logits again (with the same arithmetic).
-        const int end = Vp - ((Vp - first) & 3), head = first < 0 ? min(first + 4, Vp) : 0;
-        const int c = tid < 4 ? tid : max(end, head) + tid - 4;
-        if (tid < 4 ? c < head : c < Vp && tid < 8)
-            p[c] = c < V ? __builtin_amdgcn_exp2f(x[c] * LOG2E - ml) * inv : 0.0f;
+        const int end = Vp - (((unsigned)Vp - first) & 3), head = first < 0 ? first + 4 : 0;
+        const int at = tid < 4 ? 0 : max(end, head), e = tid & 3;
+        if (tid < 8 && e < (tid < 4 ? head : Vp - at))
+            p[at + e] = at + e < V ? __builtin_amdgcn_exp2f(x[at + e] * LOG2E - ml) * inv : 0.0f;
     }
     if (tid == 0) {
         if (tgt >= V && tgt < Vp) losses[row] = xent_loss(0.0f);
@@ -1229,7 +1233,8 @@ void softmax_crossentropy_forward(float *probs, float *losses, const float *logi
 void crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets,
                                    int N, int V, int Vp, float dloss_scale) {
     if (N <= 0 || Vp <= 0) return;
-    const int nb = ceil_div(ceil_div(Vp + (Vp % 4 == 0 ? 0 : 3), 4), NT);
+    // (A row's chunks: Vp / 4, or, starting up to 3 columns early, as many as Vp + 3 take.)
+    const int nb = ceil_div(Vp % 4 == 0 ? Vp / 4 : (int)((Vp + 6u) / 4), NT);
     const bool nt = (size_t)N * Vp * sizeof(float) >= STREAM_BYTES;
     // Rows per launch: a dispatch holds fewer than 2^32 lanes.
     const int rows = (int)std::max(1LL, ((1LL << 32) - 1) / NT / nb);

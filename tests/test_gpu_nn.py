@@ -281,6 +281,40 @@ def test_softmax_more_rows_than_one_launch_holds(gpu):
     assert np.abs(l[same] - np.log(V)).max() < TOL * np.log(V)
 
 
+@pytest.mark.parametrize("Vp", [2 ** 31 - 4, 2 ** 31 - 1])
+def test_softmax_crossentropy_at_the_widest_rows(gpu, Vp):
+    """Rows whose last chunk of four columns ends at or past the largest int:
+    the forward of 5000 logits (all columns beyond are padding to clear) and,
+    from 0.25 everywhere, the backward of all but the last two columns."""
+    print("widest rows Vp=%d" % Vp, flush=True)
+    V = 5000
+    buf = torch.full((Vp + 128,), 7.0, dtype=torch.float32, device="cuda")
+    row = buf[64:64 + Vp]
+    logits = _f32(_rng(19).standard_normal((1, V)) * 3)
+    row[:V] = dev(logits[0])
+    d_tg = _itok([17])
+    losses = Guarded(1, poison=True)
+    bmb.call("softmax_crossentropy_forward", row.data_ptr(), losses.ptr, row.data_ptr(),
+             d_tg.data_ptr(), 1, V, Vp)
+    sync("softmax_crossentropy_forward")
+    rp, rl = O.softmax_xent_fwd(logits, np.array([17], np.int32), 1, V, V)
+    assert _nw(row[:V].cpu().numpy(), rp[0]) < TOL
+    assert np.abs(losses.get() - rl).max() < TOL * np.abs(rl).max()
+    assert not bool((row[V:] != 0).any())
+    row.fill_(0.25)
+    V, target = Vp - 2, Vp - 3
+    d_tg = _itok([target])
+    bmb.call("crossentropy_softmax_backward", row.data_ptr(), row.data_ptr(), d_tg.data_ptr(), 1,
+             V, Vp, 0.5)
+    sync("crossentropy_softmax_backward")
+    assert row[target].item() == -0.375 and not bool(row[V:].any())
+    row[target] = 0.125
+    assert not bool((row[:V] != 0.125).any())
+    assert not bool((buf[:64] != 7.0).any() or (buf[64 + Vp:] != 7.0).any())
+    del buf, row
+    torch.cuda.empty_cache()
+
+
 def test_softmax_crossentropy_bad_targets_give_nan(gpu):
     N, V, Vp = 4, 10, 12
     logits = _f32(_rng(7).standard_normal((N, Vp)))
