@@ -72,28 +72,30 @@ inline unsigned grid_for(long long items) {
 }
 
 // Columns c..c+3 (c >= -3) of a row of C: whole, or (RAG) those of them that
-// exist, the others as `fill`. (c + 3 may pass the largest int: c is compared
-// with C - 3.)
+// exist, the others as `fill`. Compared as unsigned: c + 3 may pass the largest
+// int.
 template <bool RAG>
 __device__ __forceinline__ float4 ld_cols(const float *row, int c, int C, float fill) {
-    if (!RAG || (c >= 0 && c < C - 3)) return ldu4(row + c);
+    const unsigned u = c, w = C;
+    if (!RAG || (c >= 0 && u + 3 < w)) return ldu4(row + c);
     float4 v = make_float4(fill, fill, fill, fill);
-    if (c >= 0 && c < C) v.x = row[c];
-    if (c >= -1 && c < C - 1) v.y = row[c + 1];
-    if (c >= -2 && c < C - 2) v.z = row[c + 2];
-    if (c >= -3 && c < C - 3) v.w = row[c + 3];
+    if (u + 0 < w) v.x = row[c + 0];
+    if (u + 1 < w) v.y = row[c + 1];
+    if (u + 2 < w) v.z = row[c + 2];
+    if (u + 3 < w) v.w = row[c + 3];
     return v;
 }
 template <bool RAG>
 __device__ __forceinline__ void st_cols(float *row, int c, int C, float4 v) {
-    if (!RAG || (c >= 0 && c < C - 3)) {
+    const unsigned u = c, w = C;
+    if (!RAG || (c >= 0 && u + 3 < w)) {
         stu4(row + c, v);
         return;
     }
-    if (c >= 0 && c < C) row[c] = v.x;
-    if (c >= -1 && c < C - 1) row[c + 1] = v.y;
-    if (c >= -2 && c < C - 2) row[c + 2] = v.z;
-    if (c >= -3 && c < C - 3) row[c + 3] = v.w;
+    if (u + 0 < w) row[c + 0] = v.x;
+    if (u + 1 < w) row[c + 1] = v.y;
+    if (u + 2 < w) row[c + 2] = v.z;
+    if (u + 3 < w) row[c + 3] = v.w;
 }
 
 // ------------------------------------------------------------ row/column maps
@@ -701,22 +703,31 @@ __global__ __launch_bounds__(NT) void bias_fwd_k(float *out, const float *bias, 
 }
 
 // dlogits[r, i] = (probs[r, i] - [i == target]) * scale for i < V, 0 beyond.
-// nb workgroups per row (the row is uniform: no division per lane), one chunk
-// of four columns per lane (four chunks: 618 instead of 532 us at 8192 x
-// 50304). RAG: Vp % 4 != 0; a row's chunks then start at the columns that are
-// 16-byte aligned in it, so all but its first and last are still moved by
-// aligned 128-bit accesses (2048 x 50257: 281 -> 133 us). nt: streaming
-// stores, for results that do not fit the last-level cache anyway.
-template <bool RAG>
+// One chunk of four columns per lane (four chunks: 618 instead of 532 us at
+// 8192 x 50304). RAG: Vp % 4 != 0; a row's chunks then start at the columns
+// that are 16-byte aligned in it, so all but its first and last are still moved
+// by aligned 128-bit accesses. nt: streaming stores (STREAM_BYTES).
+// per: FLAT, a row's chunks, which lane i of the launch divides into row and
+// chunk; otherwise a row's workgroups (the row is uniform).
+template <bool RAG, bool FLAT>
 __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *probs,
-                                                  const int *targets, int V, int Vp, int nb,
-                                                  float scale, bool nt) {
-    const int r = blockIdx.x / nb, part = blockIdx.x % nb;
+                                                  const int *targets, int N, int V, int Vp,
+                                                  unsigned per, float scale, bool nt) {
+    unsigned r, k;  // row, chunk of it
+    if (FLAT) {
+        const unsigned i = blockIdx.x * NT + threadIdx.x;
+        r = i / per;
+        k = i - r * per;
+        if (r >= (unsigned)N) return;
+    } else {
+        r = blockIdx.x / per;
+        k = blockIdx.x % per * NT + threadIdx.x;
+    }
     const int tgt = targets[r];
     const float *p = probs + (size_t)r * Vp;
     float *d = dlogits + (size_t)r * Vp;
     const int first = RAG ? -(int)(((size_t)r * Vp) & 3) : 0;
-    const unsigned c3 = (part * NT + threadIdx.x) * 4 + (first + 3);  // c + 3, as unsigned
+    const unsigned c3 = k * 4 + (first + 3);  // c + 3, as unsigned
     if (c3 >= Vp + 3u) return;
     const int c = (int)(c3 - 3);
     const float4 v = ld_cols<RAG>(p, c, Vp, 0.0f);
@@ -726,7 +737,7 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *pr
     o.y = c < V - 1 ? (v.y - (hit == 1 ? 1.0f : 0.0f)) * scale : 0.0f;
     o.z = c < V - 2 ? (v.z - (hit == 2 ? 1.0f : 0.0f)) * scale : 0.0f;
     o.w = c < V - 3 ? (v.w - (hit == 3 ? 1.0f : 0.0f)) * scale : 0.0f;
-    if (RAG && (c < 0 || c >= Vp - 3))
+    if (RAG && (c < 0 || (unsigned)c + 3 >= (unsigned)Vp))
         st_cols<true>(d, c, Vp, o);
     else if (nt)
         stu4_nt(d + c, o);
@@ -1233,17 +1244,27 @@ void softmax_crossentropy_forward(float *probs, float *losses, const float *logi
 void crossentropy_softmax_backward(float *dlogits, const float *probs, const int *targets,
                                    int N, int V, int Vp, float dloss_scale) {
     if (N <= 0 || Vp <= 0) return;
-    // (A row's chunks: Vp / 4, or, starting up to 3 columns early, as many as Vp + 3 take.)
-    const int nb = ceil_div(Vp % 4 == 0 ? Vp / 4 : (int)((Vp + 6u) / 4), NT);
-    const bool nt = (size_t)N * Vp * sizeof(float) >= STREAM_BYTES;
+    // A row's chunks: Vp / 4, or, starting up to 3 columns early, as many as Vp + 3 take.
+    const bool rag = Vp % 4 != 0, nt = (size_t)N * Vp * sizeof(float) >= STREAM_BYTES;
+    const int chunks = rag ? (int)((Vp + 6u) / 4) : Vp / 4, nb = ceil_div(chunks, NT);
+    // Whole workgroups per row spare the ragged kernel the division (16384 x 5001:
+    // 109 against 112 us, 2048 x 50257: 138 against 143), but idle the last one's
+    // rest: 16384 x 2501 (626 of 768 lanes) still takes 51 against 54 us, x 257 (65
+    // of 256) 9.5 against 6.3. Aligned rows, whose chunks cost less, are flat at
+    // every width (16384 x 128: 3.3 against 5.9 us, x 12300: 254 against 280; at
+    // worst 8192 x 50304: 528 against 522).
+    const bool flat = !rag || (long long)chunks * 5 < 4LL * nb * NT;
+    const int per = flat ? chunks : nb;
     // Rows per launch: a dispatch holds fewer than 2^32 lanes.
-    const int rows = (int)std::max(1LL, ((1LL << 32) - 1) / NT / nb);
-    for (int r = 0; r < N; r += rows) {
+    const long long lanes = flat ? chunks : (long long)nb * NT;
+    const int rows = (int)std::min((long long)N, ((1LL << 32) - NT) / lanes);
+    for (int r = 0; r < N; r += std::min(rows, N - r)) {
         const size_t off = (size_t)r * Vp;
-        const bool rag = Vp % 4 != 0;
-        bmb::launch(rag ? xent_bwd_k<true> : xent_bwd_k<false>,
-                    dim3((unsigned)std::min(rows, N - r) * nb), dim3(NT), 0, nullptr,
-                    dlogits + off, probs + off, targets + r, V, Vp, nb, dloss_scale, nt);
+        const int n = std::min(rows, N - r);
+        bmb::launch(rag ? flat ? xent_bwd_k<true, true> : xent_bwd_k<true, false>
+                        : xent_bwd_k<false, true>,
+                    dim3(grid_for(n * lanes)), dim3(NT), 0, nullptr, dlogits + off, probs + off,
+                    targets + r, n, V, Vp, (unsigned)per, dloss_scale, nt);
     }
 }
 

@@ -187,7 +187,10 @@ def test_bias(gpu, N, C):
 @pytest.mark.parametrize("N,V,Vp", [(256, 65, 128), (64, 50257, 50304), (17, 3000, 3001),
                                     (5, 70000, 70004), (9, 1, 4), (33, 1000, 1000),
                                     (37, 50257, 50257), (9, 1021, 1021), (7, 1022, 1025),
-                                    (5, 65533, 65534), (6, 3, 5), (5, 2, 3)])
+                                    (5, 65533, 65534), (6, 3, 5), (5, 2, 3),
+                                    # the backward's flat map of aligned rows, and both maps of ragged ones
+                                    (1000, 127, 128), (33, 1100, 1100), (1000, 65, 65), (301, 257, 257),
+                                    (70, 1537, 1537), (70, 1791, 1791), (70, 1793, 1795)])
 def test_softmax_crossentropy(gpu, N, V, Vp):
     r = _rng(6)
     logits = _f32(r.standard_normal((N, Vp)) * 3)
