@@ -19,6 +19,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "launch.hpp"
@@ -71,27 +72,46 @@ inline unsigned grid_for(long long items) {
     return (unsigned)((items + NT - 1) / NT);
 }
 
-// Columns c..c+3 (c >= -3) of a row of C: whole, or (RAG) those of them that
-// exist, the others as `fill`. Compared as unsigned: c + 3 may pass the largest
-// int.
+// Columns c..c+3 of a row of C: whole, or (RAG) those of them that exist, the
+// others as `fill`.
 template <bool RAG>
 __device__ __forceinline__ float4 ld_cols(const float *row, int c, int C, float fill) {
+    if (!RAG || (c >= 0 && c + 3 < C)) return ldu4(row + c);
+    float4 v = make_float4(fill, fill, fill, fill);
+    if (c + 0 >= 0 && c + 0 < C) v.x = row[c + 0];
+    if (c + 1 >= 0 && c + 1 < C) v.y = row[c + 1];
+    if (c + 2 >= 0 && c + 2 < C) v.z = row[c + 2];
+    if (c + 3 >= 0 && c + 3 < C) v.w = row[c + 3];
+    return v;
+}
+template <bool RAG>
+__device__ __forceinline__ void st_cols(float *row, int c, int C, float4 v) {
+    if (!RAG || (c >= 0 && c + 3 < C)) {
+        stu4(row + c, v);
+        return;
+    }
+    if (c + 0 >= 0 && c + 0 < C) row[c + 0] = v.x;
+    if (c + 1 >= 0 && c + 1 < C) row[c + 1] = v.y;
+    if (c + 2 >= 0 && c + 2 < C) row[c + 2] = v.z;
+    if (c + 3 >= 0 && c + 3 < C) row[c + 3] = v.w;
+}
+// The same for rows as wide as an int reaches (c + 3 may pass it; c >= -3),
+// compared as unsigned. (Of several ways to write the bound this one costs the
+// ragged cross-entropy backward nothing, others 8%; here, in place of the
+// above, it cost the token-embedding gradient 10% at 8192 positions x 65.)
+template <bool RAG>
+__device__ __forceinline__ float4 ld_cols_wide(const float *row, int c, int C) {
     const unsigned u = c, w = C;
     if (!RAG || (c >= 0 && u + 3 < w)) return ldu4(row + c);
-    float4 v = make_float4(fill, fill, fill, fill);
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (u + 0 < w) v.x = row[c + 0];
     if (u + 1 < w) v.y = row[c + 1];
     if (u + 2 < w) v.z = row[c + 2];
     if (u + 3 < w) v.w = row[c + 3];
     return v;
 }
-template <bool RAG>
-__device__ __forceinline__ void st_cols(float *row, int c, int C, float4 v) {
+__device__ __forceinline__ void st_cols_wide(float *row, int c, int C, float4 v) {
     const unsigned u = c, w = C;
-    if (!RAG || (c >= 0 && u + 3 < w)) {
-        stu4(row + c, v);
-        return;
-    }
     if (u + 0 < w) row[c + 0] = v.x;
     if (u + 1 < w) row[c + 1] = v.y;
     if (u + 2 < w) row[c + 2] = v.z;
@@ -158,21 +178,26 @@ __global__ __launch_bounds__(NT) void encoder_bwd_wpe_k(float *dwpe, const float
 // occurrence in order and owns the update of that wte row, so no two waves
 // touch the same row. What bounds it is the pass over the ids: a chain of
 // dependent loads where few tokens own many positions, and instructions where
-// most positions are a token's only one. So it takes WTE_IDS ids at a time
+// most positions are a token's only one. So it takes 256 Q ids at a time
 // with 128-bit loads, and only where it finds the token lists the positions in
 // LDS, in ascending order, and loads their rows eight at a time. (64 ids and
-// one row per step took 53 us at 4096 positions of 65 tokens x 384, 88 us at
-// 8192 of 50257 x 768 and 7.3 ms where all 8192 are one token; now 21, 58 and 1200 us.)
-constexpr int WTE_IDS = 1024;
+// one row per step took 53 us at 4096 positions of 65 tokens x 384, 81 us at
+// 8192 of 50257 x 768 and 7.3 ms where all 8192 are one token; now 21, 52 and
+// 1200 us.) Q is 4, or 1 up to WTE_FEW positions, where most of a step of 1024
+// is past the end (us, Q = 1 against 4: 128 positions x 128 5.5 and 6.3, 512 x
+// 768 7.1 and 7.7; 1024 x 128 10.6 and 9.8). Rows of odd width take strips as
+// wide as the others (8192 x 767 of 50257: 71 us in strips of 768, 105 of 256).
+constexpr int WTE_FEW = 512;
 
 // ids[k] = the lane's ids tokens[j0 + 256 k + 4 lane + 0..3], `other` from
 // position `end` on.
-__device__ __forceinline__ void load_ids(int4 (&ids)[WTE_IDS / 256], const int *tokens, int j0,
-                                         int end, int other, int lane) {
+template <int Q>
+__device__ __forceinline__ void load_ids(int4 (&ids)[Q], const int *tokens, int j0, int end,
+                                         int other, int lane) {
     const int *p = tokens + j0 + 4 * lane;
 #pragma unroll
-    for (int k = 0; k < WTE_IDS / 256; ++k) {
-        if (j0 + WTE_IDS <= end) {
+    for (int k = 0; k < Q; ++k) {
+        if (j0 + 256 * Q <= end) {
             __builtin_memcpy(&ids[k], p + 256 * k, sizeof(int4));
         } else {
             const int left = end - (j0 + 4 * lane + 256 * k);
@@ -183,24 +208,25 @@ __device__ __forceinline__ void load_ids(int4 (&ids)[WTE_IDS / 256], const int *
         }
     }
 }
-__device__ __forceinline__ bool any_is(const int4 (&ids)[WTE_IDS / 256], int tok) {
+template <int Q>
+__device__ __forceinline__ bool any_is(const int4 (&ids)[Q], int tok) {
     bool hit = false;
 #pragma unroll
-    for (int k = 0; k < WTE_IDS / 256; ++k)
+    for (int k = 0; k < Q; ++k)
         hit |= ids[k].x == tok || ids[k].y == tok || ids[k].z == tok || ids[k].w == tok;
     return __ballot(hit) != 0;
 }
 
-template <int NCH, bool VEC>
+template <int NCH, bool VEC, int Q>
 __global__ __launch_bounds__(NT) void encoder_bwd_wte_k(float *dwte, const float *dout,
                                                          const int *tokens, int N, int C) {
-    __shared__ int found[NT / 64][WTE_IDS];
+    __shared__ int found[NT / 64][256 * Q];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i = blockIdx.x * (NT / 64) + wave;
     if (i >= N) return;
     const int tok = __builtin_amdgcn_readfirstlane(tokens[i]);
-    int4 ids[WTE_IDS / 256];
-    for (int j0 = 0; j0 < i; j0 += WTE_IDS) {
+    int4 ids[Q];
+    for (int j0 = 0; j0 < i; j0 += 256 * Q) {
         load_ids(ids, tokens, j0, i, ~tok, lane);
         if (any_is(ids, tok)) return;
     }
@@ -209,13 +235,13 @@ __global__ __launch_bounds__(NT) void encoder_bwd_wte_k(float *dwte, const float
     float4 s[NCH];
 #pragma unroll
     for (int h = 0; h < NCH; ++h) s[h] = zero4();
-    for (int j0 = i; j0 < N; j0 += WTE_IDS) {
+    for (int j0 = i; j0 < N; j0 += 256 * Q) {
         load_ids(ids, tokens, j0, N, ~tok, lane);
         if (!any_is(ids, tok)) continue;
         int n = 0;
         const unsigned long long below = (1ULL << lane) - 1;
 #pragma unroll
-        for (int k = 0; k < WTE_IDS / 256; ++k) {
+        for (int k = 0; k < Q; ++k) {
             const int id[4] = {ids[k].x, ids[k].y, ids[k].z, ids[k].w};
             int at = n;
 #pragma unroll
@@ -738,7 +764,7 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *pr
     const unsigned c3 = k * 4 + (first + 3);  // c + 3, as unsigned
     if (c3 >= Vp + 3u) return;
     const int c = (int)(c3 - 3);
-    const float4 v = ld_cols<RAG>(p, c, Vp, 0.0f);
+    const float4 v = ld_cols_wide<RAG>(p, c, Vp);
     const unsigned hit = (unsigned)tgt - (unsigned)c;  // the target's place in the chunk
     float4 o;
     o.x = c < V - 0 ? (v.x - (hit == 0 ? 1.0f : 0.0f)) * scale : 0.0f;
@@ -746,7 +772,7 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(float *dlogits, const float *pr
     o.z = c < V - 2 ? (v.z - (hit == 2 ? 1.0f : 0.0f)) * scale : 0.0f;
     o.w = c < V - 3 ? (v.w - (hit == 3 ? 1.0f : 0.0f)) * scale : 0.0f;
     if (RAG && (c < 0 || (unsigned)c + 3 >= (unsigned)Vp))
-        st_cols<true>(d, c, Vp, o);
+        st_cols_wide(d, c, Vp, o);
     else if (nt)
         stu4_nt(d + c, o);
     else
@@ -1160,14 +1186,17 @@ void encoder_backward(float *dwte, float *dwpe, const float *dout, const int *to
         bmb::launch(encoder_bwd_wpe_k<false>, dim3(grid_for(items)), dim3(NT), 0, nullptr,
                     dwpe, dout, B, T, C, C4, items);
     const int N = B * T;
-    auto wte = [&](auto kern, int nch) {
-        bmb::launch(kern, dim3(ceil_div(N, NT / 64), ceil_div(C, 256 * nch)), dim3(NT), 0, nullptr,
-                    dwte, dout, tokens, N, C);
+    const bool vec = C % 4 == 0, few = N <= WTE_FEW;
+    auto wte = [&](auto nch) {
+        constexpr int NC = decltype(nch)::value;
+        bmb::launch(vec ? few ? encoder_bwd_wte_k<NC, true, 1> : encoder_bwd_wte_k<NC, true, 4>
+                        : few ? encoder_bwd_wte_k<NC, false, 1> : encoder_bwd_wte_k<NC, false, 4>,
+                    dim3(ceil_div(N, NT / 64), ceil_div(C, 256 * NC)), dim3(NT), 0, nullptr, dwte,
+                    dout, tokens, N, C);
     };
-    if (C % 4 != 0) wte(encoder_bwd_wte_k<1, false>, 1);
-    else if (C <= 256) wte(encoder_bwd_wte_k<1, true>, 1);
-    else if (C <= 512) wte(encoder_bwd_wte_k<2, true>, 2);
-    else wte(encoder_bwd_wte_k<3, true>, 3);
+    if (C <= 256) wte(std::integral_constant<int, 1>{});
+    else if (C <= 512) wte(std::integral_constant<int, 2>{});
+    else wte(std::integral_constant<int, 3>{});
 }
 
 void layernorm_forward(float *out, float *mean, float *rstd, const float *inp,

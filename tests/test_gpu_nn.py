@@ -77,6 +77,29 @@ def test_encoder(gpu, B, T, C, V):
     assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
 
 
+# Ids that mostly occur once (every position owns a row), one that occurs at the
+# ends of the steps the ids are read in, on both sides of the step sizes and of
+# each width of strip, even and odd.
+@pytest.mark.parametrize("B,T,C,V", [(8, 1024, 768, 50304), (4, 128, 300, 3000), (1, 513, 767, 5000),
+                                     (1, 2049, 513, 50257), (3, 85, 255, 1000), (1, 1025, 385, 900)])
+def test_encoder_backward_of_mostly_distinct_ids(gpu, B, T, C, V):
+    r = _rng(11)
+    N = B * T
+    tok = r.integers(0, V, N).astype(np.int32)
+    tok[[j for j in (0, 255, 256, 511, 512, 1023, 1024, N - 1) if j < N]] = V - 1
+    print("encoder backward B=%d T=%d C=%d V=%d" % (B, T, C, V), flush=True)
+    dout = _f32(r.standard_normal((N, C)))
+    dwte0, dwpe0 = _f32(r.standard_normal(V * C)), _f32(r.standard_normal(T * C))
+    dwte, dwpe = Guarded(V * C, fill=dwte0), Guarded(T * C, fill=dwpe0)
+    d_dout, d_tok = dev(dout), _itok(tok)
+    bmb.call("encoder_backward", dwte.ptr, dwpe.ptr, d_dout.data_ptr(), d_tok.data_ptr(), B, T, C)
+    sync("encoder_backward")
+    assert dwte.ok() and dwpe.ok()
+    rw, rp = O.encoder_bwd(dwte0, dwpe0, dout, tok, B, T, C)
+    assert _nw(dwte.get() - dwte0, rw - dwte0) < TOL
+    assert _nw(dwpe.get() - dwpe0, rp - dwpe0) < TOL
+
+
 @pytest.mark.parametrize("N,C", [(256, 128), (8192, 768), (37, 1024), (50, 100), (9, 1536),
                                  (5, 4), (3, 1), (70, 255), (41, 1025), (33, 1599), (19, 2048),
                                  (6, 2051)])
