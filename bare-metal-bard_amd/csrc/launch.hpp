@@ -4,8 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <map>
 #include <mutex>
-#include <set>
 #include <utility>
 
 #include "status.hpp"
@@ -13,8 +13,10 @@
 namespace bmb {
 
 // Kernels whose dynamic LDS exceeds the 64 KiB default get their limit raised
-// once per kernel and device (gfx950 has 160 KiB per CU). Keyed on the
-// kernel's address: kernels of one signature share this instantiation.
+// to the most a launch on that device has asked for (gfx950 has 160 KiB per
+// CU); a kernel whose LDS grows with the problem (the layernorm backward) asks
+// again. Keyed on the kernel's address: kernels of one signature share this
+// instantiation.
 template <typename K>
 inline void allow_smem(K kern, size_t bytes) {
     if (bytes <= 65536) return;
@@ -22,9 +24,11 @@ inline void allow_smem(K kern, size_t bytes) {
     if (hipGetDevice(&dev) != hipSuccess) return;
     const void *f = reinterpret_cast<const void *>(kern);
     static std::mutex mu;
-    static std::set<std::pair<int, const void *>> done;
+    static std::map<std::pair<int, const void *>, size_t> limits;
     std::lock_guard<std::mutex> lock(mu);  // held until the attribute is set
-    if (!done.insert({dev, f}).second) return;
+    size_t &limit = limits[{dev, f}];
+    if (bytes <= limit) return;
+    limit = bytes;
     note_launch_status(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)bytes));
 }
