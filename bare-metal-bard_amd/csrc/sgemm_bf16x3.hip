@@ -780,7 +780,7 @@ __global__ __launch_bounds__(Tl::NT * KS) void bf16x3_ks_k(int M, int N, int K, 
 }
 
 // Problems with an M, N or K below MIN_DIM, or too large for 32-bit offsets
-// within a tile (part_time): 64 x 64 tiles whose operands are loaded element
+// within a tile (reaches): 64 x 64 tiles whose operands are loaded element
 // by element.
 constexpr int MIN_DIM = 4;
 template <bool TA, bool TB, int EPI>
@@ -949,11 +949,21 @@ const Device &device_info(int dev) {
     return info[dev];
 }
 
-// What a plan depends on besides M, N and K: the transposes, and whether an
-// operand's rows are not 16-byte aligned.
+// What a plan depends on besides M, N and K: the transposes, whether an
+// operand's rows are not 16-byte aligned, and the stored row strides (a band's
+// operands keep those of the whole problem).
 struct Layout {
     bool ta, tb, mis_a, mis_b;
+    int lda, ldb;
 };
+
+// Whether the staging loads' byte offsets within a tile (OpStage::o) stay
+// below 2^32: they span the tile's rows of an operand with contiguous k, BK
+// rows of one with contiguous m or n.
+bool reaches(const B3Cand &c, const Layout &lo) {
+    return (lo.ta ? BK + 1LL : c.bm) * lo.lda < 1LL << 30 &&
+           (lo.tb ? (long long)c.bn : BK + 1LL) * lo.ldb < 1LL << 30;
+}
 
 // Modelled time (us) of an M x N x K band on tile t with K split s ways;
 // false if that split is not allowed (may_split, max_floats caps splits * M *
@@ -961,10 +971,6 @@ struct Layout {
 bool part_time(const Device &dv, int M, int N, int K, int t, int s, Layout lo, bool may_split,
                long long max_floats, Part &out, double &time) {
     const B3Cand &c = CANDS[t];
-    // The staging loads' byte offsets within a tile stay below 2^32.
-    if (std::max(c.bm, c.bn) * (long long)K >= 1LL << 30 ||
-        (BK + 1LL) * std::max(M, N) >= 1LL << 30)
-        return false;
     int splits = 1, kchunk = K;
     if (c.ks > 1) {
         if (K / s < c.ks * MIN_SLICE_K) return false;
@@ -1001,15 +1007,20 @@ bool part_time(const Device &dv, int M, int N, int K, int t, int s, Layout lo, b
 }
 
 // The fastest single-band plan of an M x N x K band (split K ranges of at
-// least min_split_k; k-sliced tiles only if ks_ok).
+// least min_split_k; k-sliced tiles only if ks_ok). Where no tile reaches, or
+// a dimension is below MIN_DIM, the narrow kernel, planned as the 64 x 64 tile.
 double best_part(const Device &dv, int M, int N, int K, Layout lo, bool may_split,
                  long long max_floats, Part &best, int min_split_k = 0, bool ks_ok = false) {
     double best_t = -1.0;
-    const bool narrow = std::min({M, N, K}) < MIN_DIM;
+    bool narrow = std::min({M, N, K}) < MIN_DIM;
+    if (!narrow) {
+        narrow = true;
+        for (const B3Cand &c : CANDS) narrow &= !(reaches(c, lo) && (c.ks == 1 || ks_ok));
+    }
     best = Part{NARROW, 1, K};
     for (int t = 0; t < N_CANDS; ++t)
         for (int s : SPLITS) {
-            if ((CANDS[t].ks > 1 && !ks_ok) || (narrow && t != 2)) continue;
+            if ((CANDS[t].ks > 1 && !ks_ok) || (narrow ? t != 2 : !reaches(CANDS[t], lo))) continue;
             Part p;
             double tm;
             if (part_time(dv, M, N, K, t, s, lo, may_split, max_floats, p, tm) &&
@@ -1019,7 +1030,6 @@ double best_part(const Device &dv, int M, int N, int K, Layout lo, bool may_spli
                 if (narrow) best.tile = NARROW;
             }
         }
-    if (best_t < 0) best_t = 1e12;  // no tile reaches: NARROW, whatever it takes
     return best_t;
 }
 
@@ -1034,7 +1044,7 @@ Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long
     // Two bands: the first whole rounds of one tile, the rest on its own plan.
     for (int t = 0; K >= MIN_BAND_K && std::min(M, N) >= MIN_DIM && t < N_CANDS; ++t) {
         const B3Cand &c = CANDS[t];
-        if (c.ks > 1) continue;
+        if (c.ks > 1 || !reaches(c, lo)) continue;
         const long long tiles_n = bmb::ceil_div(N, c.bn);
         const long long slots = (long long)dv.cus * dv.occ[t];
         for (long long k = 1;; ++k) {
@@ -1060,7 +1070,7 @@ Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long
     // scratch only where K may be split).
     for (int t = 0; edges_ok && may_split && K >= MIN_CORNER_K && t < N_CANDS; ++t) {
         const B3Cand &c = CANDS[t];
-        if (c.ks > 1) continue;
+        if (c.ks > 1 || !reaches(c, lo)) continue;
         const int m1 = M / c.bm * c.bm, n1 = N / c.bn * c.bn;
         if (m1 == 0 || n1 == 0 || (m1 == M && n1 == N) || M - m1 > bmb::EDGE_MAX ||
             N - n1 > bmb::EDGE_MAX || bmb::edge_partial_floats(M - m1, N - n1, N, K) > max_floats)
@@ -1269,7 +1279,7 @@ bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const 
     // same bits.)
     const bool ks_ok = true;
     const Layout lo{ta, tb, (ta ? M : K) % 4 != 0 || ((uintptr_t)A & 15) != 0,
-                    (tb ? K : N) % 4 != 0 || ((uintptr_t)B & 15) != 0};
+                    (tb ? K : N) % 4 != 0 || ((uintptr_t)B & 15) != 0, ta ? M : K, tb ? K : N};
     Plan p = pick(M, N, K, lo, may_split, fixed ? fixed_floats : MAX_SPLIT_FLOATS,
                   edges_ok, ks_ok);
     float *P = fixed;
