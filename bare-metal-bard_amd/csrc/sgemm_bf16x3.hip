@@ -204,9 +204,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t operand(const float *p) {
 // (load_tail) fills with zeros. Every path loads whole vectors and selects
 // from them afterwards: where a branch joined vectors loaded at once with
 // vectors loaded element by element, the compiler (ROCm 7.2) reused registers
-// of the former that were still live. That needs at least W rows and k, and
-// byte offsets below 2^32; EW (bf16x3_narrow_k) loads every element by itself.
-template <int ROWS, int NT, bool KCONT, bool IN, bool EW = false>
+// of the former that were still live. That needs stored rows of at least four
+// elements and byte offsets below 2^32.
+//
+// SHORT: stored rows may be shorter (a K below 4 with k contiguous, an M or N
+// below 4 otherwise), down to four elements in the whole operand. A vector then
+// runs on into the next stored row, whose elements are masked (k) or only reach
+// outputs that are not stored (rows); near the operand's end it is loaded from
+// further back and shifted into place (load_tail, which also takes a whole
+// stage with fewer than SHORT_K k behind its first). SINGLE: every element is
+// loaded by itself.
+enum Stage { VECTOR, SHORT, SINGLE };
+constexpr int SHORT_K = BK + 3;  // loads of a whole stage stay inside the operand
+template <int ROWS, int NT, bool KCONT, bool IN, Stage MODE = VECTOR>
 struct OpStage {
     static constexpr int CH = ROWS * BK / 4 / NT;  // KCONT: chunks per lane
     static constexpr int W = !KCONT && ROWS * BK / 16 < NT ? 2 : 4;
@@ -223,7 +233,7 @@ struct OpStage {
     // row0(), k 0), and how many rows before its place each block is loaded:
     // loop-invariant.
     unsigned o[NLD];
-    int shift[KCONT || IN ? 1 : PER_T];
+    int shift[KCONT || IN || MODE != VECTOR ? 1 : PER_T];
 
     __device__ static __forceinline__ bool skip(int j, int tid) {
         return !KCONT && BLK % NT != 0 && tid + j * NT >= BLK;
@@ -242,7 +252,9 @@ struct OpStage {
     }
     // The row that offsets count from: the tile's first, or 0 where a clamped
     // block may start before the tile.
-    __device__ static __forceinline__ int row0(int r0) { return IN || KCONT ? r0 : 0; }
+    __device__ static __forceinline__ int row0(int r0) {
+        return (IN && MODE != SHORT) || KCONT ? r0 : 0;
+    }
     // R rows in all, ld: the stored row stride, r0: the tile's first row.
     __device__ __forceinline__ void setup(int R, int ld, int r0, int tid) {
         if constexpr (KCONT) {
@@ -258,7 +270,9 @@ struct OpStage {
             for (int j = 0; j < PER_T; ++j) {
                 int kb, rb;
                 block(min(tid + j * NT, BLK - 1), kb, rb);
-                if (!IN) {
+                if (MODE == SHORT) {
+                    rb = min(rb, R - 1 - r0);
+                } else if (!IN) {
                     shift[j] = rb - min(rb, R - r0 - W);
                     rb -= shift[j];
                 }
@@ -297,7 +311,7 @@ struct OpStage {
         for (int i = 0; i < NLD; ++i)
             if (!skip(i / 4, tid)) v[i] = ldv(p, o[i]);
     }
-    // EW: every element (row, k) by itself; rows past the last of R repeat it,
+    // SINGLE: every element (row, k) by itself; rows past the last of R repeat it,
     // k from rem (> 0) on are zeros. p: the stage's (row 0 of the operand,
     // k 0) element.
     __device__ __forceinline__ void load_single(const float *p, int R, int ld, int r0, int rem,
@@ -324,11 +338,29 @@ struct OpStage {
     // become zero. p: the descriptor of the stage's base (KCONT: of the four
     // elements before it; a chunk with fewer than four k is loaded as the
     // stage's last four and shifted).
-    __device__ __forceinline__ void load_tail(__amdgpu_buffer_rsrc_t p, int ld, int rem, int tid) {
+    // SHORT: p is the descriptor of the four elements before the stage's base,
+    // end the stored elements from that base to the operand's (or K range's)
+    // last one, and rem may be any positive number.
+    __device__ __forceinline__ void load_tail(__amdgpu_buffer_rsrc_t p, int ld, int rem, int tid,
+                                              long long end = 0) {
+        const unsigned last = (unsigned)min(4LL * (end - W + 4), 0xffffffffLL);
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             if (skip(i / 4, tid)) continue;
-            if constexpr (KCONT) {
+            if constexpr (MODE == SHORT) {
+                int k, row;
+                if (KCONT) {
+                    chunk(tid + i * NT, row, k);
+                } else {
+                    block(tid + i / 4 * NT, k, row);
+                    k = 4 * k + i % 4;
+                }
+                const unsigned at = min(o[i] + 16u, last);
+                v[i] = shifted(ldv(p, at), (int)((o[i] + 16u - at) / 4u));
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+                    v[i].f[e] = k + (KCONT ? e : 0) < rem ? v[i].f[e] : 0.0f;
+            } else if constexpr (KCONT) {
                 int r, c;
                 chunk(tid + i * NT, r, c);
                 const int n = c - min(c, rem - 4);
@@ -369,7 +401,8 @@ struct OpStage {
             float x[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                x[i] = IN || EW ? v[4 * j + i].f[c] : shifted(v[4 * j + i], shift[j]).f[c];
+                x[i] = IN || MODE != VECTOR ? v[4 * j + i].f[c]
+                                            : shifted(v[4 * j + i], shift[j]).f[c];
             split4(x, h, l);
             *reinterpret_cast<bf16x4 *>(hi + lds_off(row + c, 4 * kb)) = h;
             *reinterpret_cast<bf16x4 *>(lo + lds_off(row + c, 4 * kb)) = l;
@@ -404,10 +437,10 @@ struct Bf16x3Gemm {
     // with 128-bit loads (blocks half as wide, on all lanes for both
     // operands, halve the bytes per load).
     static constexpr bool PAIR = TA && !TB && BM == BN && BM * BK / 16 * 2 == NT;
-    template <bool IN, bool EW>
-    using StageA = OpStage<BM, PAIR ? NT / 2 : NT, !TA, IN, EW>;
-    template <bool IN, bool EW>
-    using StageB = OpStage<BN, PAIR ? NT / 2 : NT, TB, IN, EW>;
+    template <bool IN, Stage MODE>
+    using StageA = OpStage<BM, PAIR ? NT / 2 : NT, !TA, IN, MODE>;
+    template <bool IN, Stage MODE>
+    using StageB = OpStage<BN, PAIR ? NT / 2 : NT, TB, IN, MODE>;
 
     // One 16-k step of MFMAs on stage `st`: for every 32 x 32 block,
     // acc += lo_a hi_b, then hi_a lo_b, then hi_a hi_b (small terms first).
@@ -495,8 +528,8 @@ struct Bf16x3Gemm {
     // stages holds data) and every slice runs kloop stages, so that all of
     // them meet at the same barriers. The slices' sums are then added in LDS,
     // in slice order, and slice 0 runs the epilogue.
-    // EW: M, N or K may be below MIN_DIM (not INTERIOR; see OpStage).
-    template <bool INTERIOR, int EPI, bool TAIL, int KS = 1, bool EW = false>
+    // MODE: how both operands are staged (OpStage; TAIL unless VECTOR).
+    template <bool INTERIOR, int EPI, bool TAIL, int KS = 1, Stage MODE = VECTOR>
     __device__ static __forceinline__ void run(int M, int N, int K, int lda, int ldb, float alpha,
                                                const float *__restrict__ A,
                                                const float *__restrict__ B, float beta, float *C,
@@ -515,8 +548,8 @@ struct Bf16x3Gemm {
                 for (int r = 0; r < 16; ++r) acc[fi][fn][r] = 0.0f;
 
         const int nkt = KS > 1 ? kloop : (K + BK - 1) / BK;
-        using SA = StageA<INTERIOR, EW>;
-        using SB = StageB<INTERIOR, EW>;
+        using SA = StageA<INTERIOR, MODE>;
+        using SB = StageB<INTERIOR, MODE>;
         SA ga;
         SB gb;
         // PAIR: this half's operand in ga (uniform over a wave).
@@ -536,14 +569,24 @@ struct Bf16x3Gemm {
         };
         auto load = [&](int kt) {
             const int rem = K - kt * BK;
-            if (EW) {
+            if (MODE == SINGLE) {
                 const size_t k = (size_t)kt * BK;
                 ga.load_single((up ? B : A) + (TA ? k * lda1 : k), up ? N : M, lda1, a0, rem,
                                stid);
                 if (!PAIR) gb.load_single(B + (TB ? k : k * ldb), N, ldb, n0, rem, tid);
-            } else if (!TAIL || rem >= BK) {
+            } else if (!TAIL || rem >= (MODE == SHORT ? SHORT_K : BK)) {
                 ga.load(operand(a_at(kt)), stid);
                 if (!PAIR) gb.load(operand(b_at(kt)), tid);
+            } else if (MODE == SHORT && rem > 0) {
+                // Elements from each stage's base to the end of its operand's K
+                // range: whole rows of k from row0 on, or whole k of rows.
+                const auto left = [&](bool kcont, int R, int ld, int r) {
+                    return kcont ? (R - 1LL - r) * ld + rem : (rem - 1LL) * ld + R;
+                };
+                ga.load_tail(operand(a_at(kt) - 4), lda1, rem, stid,
+                             left(!TA, up ? N : M, lda1, ga.row0(a0)));
+                if (!PAIR)
+                    gb.load_tail(operand(b_at(kt) - 4), ldb, rem, tid, left(TB, N, ldb, gb.row0(n0)));
             } else if (rem > 0) {
                 ga.load_tail(operand(a_at(kt) - (TA ? 0 : 4)), lda1, rem, stid);
                 if (!PAIR) gb.load_tail(operand(b_at(kt) - (TB ? 4 : 0)), ldb, rem, tid);
@@ -570,7 +613,7 @@ struct Bf16x3Gemm {
         // spilled 24-34 of them).
         constexpr int UNROLL = Tl::SMEM_BYTES <= 98304 ? 2 : 1;
         int kt0 = 0;
-        for (const int whole = EW ? 0 : K / BK; kt0 + 1 + UNROLL < whole; kt0 += UNROLL)
+        for (const int whole = MODE == SINGLE ? 0 : MODE == SHORT ? (K - 3) / BK : K / BK; kt0 + 1 + UNROLL < whole; kt0 += UNROLL)
             static_for<0, UNROLL>([&](auto uc) {
                 const int kt = kt0 + uc, h = UNROLL == 2 ? (int)uc : kt & 1;
                 const __bf16 *st = smem + h * Tl::STAGE;
@@ -714,8 +757,8 @@ struct Bf16x3Gemm {
 // offset to its first row and column) runs as a problem of its own.
 // KT: K is not a whole number of stages. (A separate instantiation: the last
 // stage's loads cost the 256 x 256 kernels spilled registers, which the other
-// shapes need not pay.)
-template <class Tl, bool TA, bool TB, int EPI, bool KT>
+// shapes need not pay.) MODE: OpStage's; SHORT only with KT.
+template <class Tl, bool TA, bool TB, int EPI, bool KT, Stage MODE = VECTOR>
 __global__ __launch_bounds__(Tl::NT) void bf16x3_k(int M, int N, int K, int kchunk, float alpha,
                                                    const float *__restrict__ A, int lda,
                                                    const float *__restrict__ B, int ldb,
@@ -732,11 +775,11 @@ __global__ __launch_bounds__(Tl::NT) void bf16x3_k(int M, int N, int K, int kchu
     float *Cs = EPI == bmb::EPI_PARTIAL ? C + (size_t)blockIdx.y * M * N : C;
     const int ldcs = EPI == bmb::EPI_PARTIAL ? N : ldc;
     if (m0 + Tl::BM <= M && n0 + Tl::BN <= N)
-        G::template run<true, EPI, KT>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0, n0,
-                                       lds, ep);
+        G::template run<true, EPI, KT, 1, MODE>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs,
+                                                ldcs, m0, n0, lds, ep);
     else
-        G::template run<false, EPI, KT>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs, m0,
-                                        n0, lds, ep);
+        G::template run<false, EPI, KT, 1, MODE>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs,
+                                                 ldcs, m0, n0, lds, ep);
 }
 
 // The same tile as KS k-slices of Tl::NT lanes each: every slice runs per =
@@ -746,7 +789,7 @@ __global__ __launch_bounds__(Tl::NT) void bf16x3_k(int M, int N, int K, int kchu
 // device, where split-K alone would need a second launch for its reduce or
 // many more ranges (and partials) for the same number of waves.
 // KT: some slice's range is not `per` whole stages.
-template <class Tl, bool TA, bool TB, int EPI, int KS, bool KT>
+template <class Tl, bool TA, bool TB, int EPI, int KS, bool KT, Stage MODE = VECTOR>
 __global__ __launch_bounds__(Tl::NT * KS) void bf16x3_ks_k(int M, int N, int K, int kchunk,
                                                            float alpha,
                                                            const float *__restrict__ A, int lda,
@@ -772,17 +815,15 @@ __global__ __launch_bounds__(Tl::NT * KS) void bf16x3_ks_k(int M, int N, int K, 
     const int ldcs = EPI == bmb::EPI_PARTIAL ? N : ldc;
     __bf16 *st = lds + (size_t)slice * 2 * Tl::STAGE;
     if (m0 + Tl::BM <= M && n0 + Tl::BN <= N)
-        G::template run<true, EPI, KT, KS>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs,
-                                             m0, n0, st, ep, per);
+        G::template run<true, EPI, KT, KS, MODE>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs,
+                                                 ldcs, m0, n0, st, ep, per);
     else
-        G::template run<false, EPI, KT, KS>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, ldcs,
-                                              m0, n0, st, ep, per);
+        G::template run<false, EPI, KT, KS, MODE>(M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs,
+                                                  ldcs, m0, n0, st, ep, per);
 }
 
-// Problems with an M, N or K below MIN_DIM, or too large for 32-bit offsets
-// within a tile (reaches): 64 x 64 tiles whose operands are loaded element
-// by element.
-constexpr int MIN_DIM = 4;
+// Problems that no other kernel takes (SINGLE): 64 x 64 tiles whose
+// operands are loaded element by element.
 template <bool TA, bool TB, int EPI>
 __global__ __launch_bounds__(TileS::NT) void bf16x3_narrow_k(int M, int N, int K, int kchunk,
                                                              float alpha,
@@ -798,7 +839,7 @@ __global__ __launch_bounds__(TileS::NT) void bf16x3_narrow_k(int M, int N, int K
     const float *Ak = TA ? A + (size_t)kb * lda : A + kb;
     const float *Bk = TB ? B + kb : B + (size_t)kb * ldb;
     float *Cs = EPI == bmb::EPI_PARTIAL ? C + (size_t)blockIdx.y * M * N : C;
-    Bf16x3Gemm<TileS, TA, TB>::template run<false, EPI, true, 1, true>(
+    Bf16x3Gemm<TileS, TA, TB>::template run<false, EPI, true, 1, SINGLE>(
         M, N, klen, lda, ldb, alpha, Ak, Bk, beta, Cs, EPI == bmb::EPI_PARTIAL ? N : ldc,
         tm * TileS::BM, tn * TileS::BN, lds, ep);
 }
@@ -851,6 +892,7 @@ constexpr B3Cand CANDS[] = {
 };
 constexpr int N_CANDS = 9;
 constexpr int NARROW = N_CANDS;  // bf16x3_narrow_k, planned as the 64 x 64 tile
+constexpr int MIN_DIM = 4;       // the least M and N of a band (vector loads of its rows)
 // The 32 x 32 tile is only taken up to XS_MAX_OUTPUTS outputs, and every
 // slice keeps at least MIN_SLICE_K of k.
 constexpr long long XS_MAX_OUTPUTS = 1LL << 20;
@@ -902,9 +944,11 @@ int ks_occupancy_of() {
                         KS * Tl::SMEM_BYTES);
 }
 
-// One band's launch: tile candidate, K ranges and the K per range.
+// One band's launch: tile candidate, K ranges, the K per range, and the
+// staging of the operands.
 struct Part {
     int tile, splits, kchunk;
+    Stage mode;
 };
 
 // Rows [0, m1) run on part[0], rows [m1, M) on part[1] (m1 == M: one band).
@@ -1002,47 +1046,68 @@ bool part_time(const Device &dv, int M, int N, int K, int t, int s, Layout lo, b
     if (splits > 1)
         time += (2.0 * splits + 1.0) * mn * 4.0 / PARTIALS_BYTES_PER_US + REDUCE_US +
                 splits * RANGE_US;
-    out = Part{t, splits, kchunk};
+    out = Part{t, splits, kchunk, VECTOR};
     return true;
 }
 
+// How an M x N x K problem's operands can be staged. Vector loads need stored
+// rows of four elements; shorter ones take the SHORT kernels (short_ok: the
+// epilogue has them) down to four elements in the whole operand. An operand
+// that is smaller still, or an empty product, is loaded element by element.
+// (An M or N below four is no short row where k is contiguous. With every
+// dimension below four loaded by element, in us, against now: 1 x 768 x 768 of
+// A B^T 9.4 and 5.9, 3 x 50257 x 768 72 and 30; SHORT: 8192 x 1 x 768 of A B
+// 14.2 and 8.3, 768 x 1 x 8192 27.0 and 11.3, 4096 x 4096 x 1 of A^T B 24.3 and
+// 14.9.)
+Stage staging(int M, int N, int K, Layout lo, bool short_ok) {
+    if (std::min(lo.lda, lo.ldb) >= MIN_DIM) return VECTOR;
+    const bool flat = (long long)M * K >= MIN_DIM && (long long)N * K >= MIN_DIM;
+    return short_ok && flat ? SHORT : SINGLE;
+}
+
+// The tiles that have a SHORT kernel.
+bool short_tile(int t) { return t == 1 || t == 2 || t == 5 || t == 7; }
+
 // The fastest single-band plan of an M x N x K band (split K ranges of at
-// least min_split_k; k-sliced tiles only if ks_ok). Where no tile reaches, or
-// a dimension is below MIN_DIM, the narrow kernel, planned as the 64 x 64 tile.
-double best_part(const Device &dv, int M, int N, int K, Layout lo, bool may_split,
+// least min_split_k; k-sliced tiles only if ks_ok). Where no tile reaches, the
+// narrow kernel.
+double best_part(const Device &dv, int M, int N, int K, Layout lo, Stage mode, bool may_split,
                  long long max_floats, Part &best, int min_split_k = 0, bool ks_ok = false) {
+    const auto usable = [&](int t) {
+        return (CANDS[t].ks == 1 || ks_ok) && (mode != SHORT || short_tile(t)) &&
+               reaches(CANDS[t], lo);
+    };
+    bool any = false;
+    for (int t = 0; t < N_CANDS; ++t) any |= usable(t);
+    if (!any) mode = SINGLE;
     double best_t = -1.0;
-    bool narrow = std::min({M, N, K}) < MIN_DIM;
-    if (!narrow) {
-        narrow = true;
-        for (const B3Cand &c : CANDS) narrow &= !(reaches(c, lo) && (c.ks == 1 || ks_ok));
-    }
-    best = Part{NARROW, 1, K};
+    best = Part{NARROW, 1, K, SINGLE};
     for (int t = 0; t < N_CANDS; ++t)
         for (int s : SPLITS) {
-            if ((CANDS[t].ks > 1 && !ks_ok) || (narrow ? t != 2 : !reaches(CANDS[t], lo))) continue;
+            if (mode == SINGLE ? t != 2 : !usable(t)) continue;
             Part p;
             double tm;
             if (part_time(dv, M, N, K, t, s, lo, may_split, max_floats, p, tm) &&
                 (p.splits == 1 || p.kchunk >= min_split_k) && (best_t < 0 || tm < best_t)) {
                 best_t = tm;
                 best = p;
-                if (narrow) best.tile = NARROW;
+                best.mode = mode;
+                if (mode == SINGLE) best.tile = NARROW;
             }
         }
     return best_t;
 }
 
-// ks_ok: the k-sliced tiles may run the problem (single-band plans only).
 Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long max_floats,
-              bool edges_ok, bool ks_ok) {
+              bool edges_ok, bool short_ok) {
     const Device &dv = device_info(dev);
-    Plan best{{Part{0, 1, K}, Part{0, 1, K}}, M, N, false};
+    const Stage mode = staging(M, N, K, lo, short_ok);
+    Plan best{{Part{0, 1, K, VECTOR}, Part{0, 1, K, VECTOR}}, M, N, false};
     const double single_t =
-        best_part(dv, M, N, K, lo, may_split, max_floats, best.part[0], 0, ks_ok);
+        best_part(dv, M, N, K, lo, mode, may_split, max_floats, best.part[0], 0, true);
     double best_t = single_t;
     // Two bands: the first whole rounds of one tile, the rest on its own plan.
-    for (int t = 0; K >= MIN_BAND_K && std::min(M, N) >= MIN_DIM && t < N_CANDS; ++t) {
+    for (int t = 0; mode == VECTOR && K >= MIN_BAND_K && t < N_CANDS; ++t) {
         const B3Cand &c = CANDS[t];
         if (c.ks > 1 || !reaches(c, lo)) continue;
         const long long tiles_n = bmb::ceil_div(N, c.bn);
@@ -1056,7 +1121,7 @@ Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long
             Part p0, p1;
             double t0, t1;
             if (!part_time(dv, m1, N, K, t, 1, lo, false, 0, p0, t0)) continue;
-            t1 = best_part(dv, M - m1, N, K, lo, may_split, max_floats, p1,
+            t1 = best_part(dv, M - m1, N, K, lo, mode, may_split, max_floats, p1,
                            MIN_BAND_SPLIT_K);
             const double tm = t0 + t1 + BAND_US;
             if (tm < BAND_GAIN * single_t && tm < best_t) {
@@ -1068,7 +1133,8 @@ Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long
     // Corner plans: whole tiles of one candidate over [0, m1) x [0, n1), the
     // edges on the edge kernels (row-major A and B, BLAS epilogue; their
     // scratch only where K may be split).
-    for (int t = 0; edges_ok && may_split && K >= MIN_CORNER_K && t < N_CANDS; ++t) {
+    for (int t = 0; mode == VECTOR && edges_ok && may_split && K >= MIN_CORNER_K && t < N_CANDS;
+         ++t) {
         const B3Cand &c = CANDS[t];
         if (c.ks > 1 || !reaches(c, lo)) continue;
         const int m1 = M / c.bm * c.bm, n1 = N / c.bn * c.bn;
@@ -1081,7 +1147,7 @@ Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long
         const double tm = t0 + 1e6 * bmb::edge_model_s(m1, N - n1, M - m1, N, K);
         if (tm < BAND_GAIN * single_t && tm < best_t) {
             best_t = tm;
-            best = Plan{{p0, Part{0, 1, K}}, m1, n1, true};
+            best = Plan{{p0, Part{0, 1, K, VECTOR}}, m1, n1, true};
         }
     }
     if (getenv("BMB_GEMM_PLAN_TRACE") != nullptr)
@@ -1101,19 +1167,19 @@ Plan plan_for(int dev, int M, int N, int K, Layout lo, bool may_split, long long
 struct PlanKey {
     int dev, M, N, K;
     Layout lo;
-    bool may_split, edges_ok, ks_ok;
+    bool may_split, edges_ok, short_ok;
     long long max_floats;
     auto tie() const { return std::tie(dev, M, N, K, lo.ta, lo.tb, lo.mis_a, lo.mis_b, may_split,
-                                       edges_ok, ks_ok, max_floats); }
+                                       edges_ok, short_ok, max_floats); }
     bool operator<(const PlanKey &o) const { return tie() < o.tie(); }
     bool operator==(const PlanKey &o) const { return tie() == o.tie(); }
 };
 
 Plan pick(int M, int N, int K, Layout lo, bool may_split, long long max_floats, bool edges_ok,
-          bool ks_ok) {
+          bool short_ok) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    const PlanKey key{dev, M, N, K, lo, may_split, edges_ok, ks_ok, max_floats};
+    const PlanKey key{dev, M, N, K, lo, may_split, edges_ok, short_ok, max_floats};
     struct Entry {
         PlanKey key;
         Plan plan;
@@ -1133,7 +1199,7 @@ Plan pick(int M, int N, int K, Layout lo, bool may_split, long long max_floats, 
             return e.plan;
         }
     }
-    const Plan p = plan_for(dev, M, N, K, lo, may_split, max_floats, edges_ok, ks_ok);
+    const Plan p = plan_for(dev, M, N, K, lo, may_split, max_floats, edges_ok, short_ok);
     std::lock_guard<std::mutex> lock(mu);
     if (memo.size() > 4096) memo.clear();
     memo.emplace(key, p);
@@ -1146,6 +1212,14 @@ struct Strides {
     int lda, ldb, ldc;
 };
 
+// Whether a tile (in KS k-slices) has a SHORT kernel (short_tile), and for this
+// epilogue: short rows are planned for gemm() only.
+template <class Tl, int KS, int EPI>
+constexpr bool HAS_SHORT = (EPI == bmb::EPI_BLAS || EPI == bmb::EPI_PARTIAL) &&
+                           ((KS == 1 && (std::is_same<Tl, TileM>::value || std::is_same<Tl, TileS>::value)) ||
+                            (KS == 4 && std::is_same<Tl, TileS>::value) ||
+                            (KS == 8 && std::is_same<Tl, TileXS>::value));
+
 template <class Tl, bool TA, bool TB, int EPI>
 void launch(int M, int N, int K, const Part &p, float alpha, const float *A, const float *B,
             float beta, float *C, const Strides &ld, hipStream_t stream, bmb::EpiArgs ep) {
@@ -1156,6 +1230,8 @@ void launch(int M, int N, int K, const Part &p, float alpha, const float *A, con
                     M, N, K, p.kchunk, alpha, A, ld.lda, B, ld.ldb, beta, C, ld.ldc, tiles_m,
                     tiles_n, ep);
     };
+    if constexpr (HAS_SHORT<Tl, 1, EPI>)
+        if (p.mode == SHORT) return go(bf16x3_k<Tl, TA, TB, EPI, true, SHORT>);
     if (K % BK != 0) go(bf16x3_k<Tl, TA, TB, EPI, true>);
     else go(bf16x3_k<Tl, TA, TB, EPI, false>);
 }
@@ -1172,6 +1248,8 @@ void launch_ks(int M, int N, int K, const Part &p, float alpha, const float *A, 
                     N, K, p.kchunk, alpha, A, ld.lda, B, ld.ldb, beta, C, ld.ldc, tiles_m,
                     tiles_n, ep);
     };
+    if constexpr (HAS_SHORT<Tl, KS, EPI>)
+        if (p.mode == SHORT) return go(bf16x3_ks_k<Tl, TA, TB, EPI, KS, true, SHORT>);
     if (p.kchunk % (BK * KS) != 0 || K % p.kchunk != 0) go(bf16x3_ks_k<Tl, TA, TB, EPI, KS, true>);
     else go(bf16x3_ks_k<Tl, TA, TB, EPI, KS, false>);
 }
@@ -1274,21 +1352,21 @@ bool bmb::bf16x3_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const 
     bmb::EpiArgs ep{bias, act, pre, nullptr};
     const bool may_split = fixed != nullptr || !bmb::stream_capturing(stream);
     const bool edges_ok = !ta && !tb && epi == bmb::EPI_BLAS;
-    // (Every epilogue has k-sliced kernels, so a fused linear layer and
-    // gemm() plus the separate bias/GELU pass plan a shape alike and give the
-    // same bits.)
-    const bool ks_ok = true;
+    // (Every epilogue has the kernels of stored rows of at least four elements,
+    // so a fused linear layer and gemm() plus the separate bias/GELU pass plan
+    // such a shape alike and give the same bits.)
+    const bool short_ok = epi == bmb::EPI_BLAS;
     const Layout lo{ta, tb, (ta ? M : K) % 4 != 0 || ((uintptr_t)A & 15) != 0,
                     (tb ? K : N) % 4 != 0 || ((uintptr_t)B & 15) != 0, ta ? M : K, tb ? K : N};
     Plan p = pick(M, N, K, lo, may_split, fixed ? fixed_floats : MAX_SPLIT_FLOATS,
-                  edges_ok, ks_ok);
+                  edges_ok, short_ok);
     float *P = fixed;
     std::optional<bmb::ScratchLease> lease;
     const long long pf = partial_floats(p, M, N, K);
     if (pf > 0 && fixed == nullptr) {
         lease.emplace(bmb::SCRATCH_GEMM, (size_t)pf * sizeof(float), stream);
         P = static_cast<float *>(lease->get());
-        if (P == nullptr) p = pick(M, N, K, lo, false, 0, edges_ok, ks_ok);  // no scratch: no split
+        if (P == nullptr) p = pick(M, N, K, lo, false, 0, edges_ok, short_ok);  // no scratch: no split
     }
     const bool banded = p.m1 < M;
     if (colsum != nullptr && p.part[0].splits == 1 && (!banded || p.part[1].splits == 1)) {

@@ -59,3 +59,17 @@ def test_offsets_that_fit_take_the_tiles(ta, tb, M, N, K):
     assert parts[0][0] != NARROW and (m1 == M or parts[1][0] != NARROW), (m1, parts)
     if K > 1 << 20:
         assert parts[0][1] > 1, parts
+
+
+# Short dimensions: only an operand of fewer than four elements (or an empty
+# product) needs the element kernel. An M (or N) below 4 is any tile's edge
+# unless it is the stored row length.
+@pytest.mark.parametrize("ta,tb,M,N,K,tiles", [
+    (0, 1, 1, 768, 768, range(NARROW)), (0, 0, 3, 50257, 768, range(NARROW)),
+    (1, 1, 2304, 2, 768, range(NARROW)), (1, 0, 768, 768, 2, range(NARROW)),
+    (0, 0, 8192, 1, 768, (1, 2, 5, 7)), (1, 0, 3, 768, 8192, (1, 2, 5, 7)),
+    (0, 1, 768, 768, 3, (1, 2, 5, 7)), (1, 1, 1, 768, 4096, (1, 2, 5, 7)),
+    (0, 0, 1, 768, 3, (NARROW,)), (0, 1, 3, 1, 2, (NARROW,)), (0, 0, 64, 64, 0, (NARROW,))])
+def test_short_dimensions(ta, tb, M, N, K, tiles):
+    m1, parts = _plan(ta, tb, M, N, K)
+    assert parts[0][0] in tiles, parts

@@ -637,13 +637,19 @@ def test_k_sliced_tiles(gpu, shape, trans, capfd, monkeypatch):
     assert e3 < bound, (e3, bound)
 
 
-# The bf16x3 kernels' edges: a dimension below 4 (elements loaded one by one);
-# rows that end inside a 4-row block, or K inside a 4-k chunk (loaded from
-# further back and shifted into place), at a multiple of 4 that is no whole
-# tile or stage, and one past one; k-slices of a split K.
+# The bf16x3 kernels' edges: rows that end inside a 4-row block, or K inside a
+# 4-k chunk (loaded from further back and shifted into place), at a multiple of
+# 4 that is no whole tile or stage, and one past one; k-slices of a split K.
 EDGE_SHAPES = [(300, 3, 130), (2, 260, 64), (130, 67, 3), (1, 1, 1), (3, 2, 1000),
                (4, 4, 4), (131, 94, 1001), (257, 66, 2051), (607, 1858, 95), (516, 388, 36),
                (64, 1024, 4096), (289, 127, 3970), (1291, 1023, 260)]
+# A dimension below 4: stored rows of 1-3 elements, with K on both sides of the
+# lengths where a whole stage is still loaded as the last ones are (32-35 k),
+# over one and several stages, tiles, k-slices and K ranges, alone and beside a
+# long operand; operands of fewer than 4 elements.
+EDGE_SHAPES += [(1, 768, 768), (3, 2304, 765), (200, 1, 33), (65, 2, 34), (129, 3, 35),
+                (70, 1, 36), (1, 70, 67), (2, 3, 68), (768, 1, 8192), (3, 770, 4099), (2, 1, 20001),
+                (1000, 1025, 1), (3, 1000, 2), (260, 2, 3), (1, 5, 3), (3, 1, 2), (1, 3, 5), (2, 2, 1)]
 
 
 @pytest.mark.parametrize("trans", TRANS, ids=_tag)
