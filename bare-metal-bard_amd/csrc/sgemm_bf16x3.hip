@@ -92,10 +92,6 @@ struct B3Tile {
     static constexpr int A_PLANE = BM * LDK, B_PLANE = BN * LDK;  // bf16 elements
     static constexpr int STAGE = 2 * A_PLANE + 2 * B_PLANE;
     static constexpr size_t SMEM_BYTES = 2 * (size_t)STAGE * sizeof(__bf16);
-    static constexpr int A_CH = BM * BK / 4 / NT;         // float4 chunks of A per lane
-    static constexpr int B_BLK = BK * BN / 16;             // 4 x 4 blocks of B per stage
-    static constexpr int B_PER_T = (B_BLK + NT - 1) / NT;  // blocks per lane
-    static_assert((BM * BK / 4) % NT == 0, "A staging splits evenly over the lanes");
     static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile is whole 32x32 blocks");
 };
 
