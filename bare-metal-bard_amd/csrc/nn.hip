@@ -5,7 +5,9 @@
 // The design rules are therefore about bytes, not flops:
 //   * each tensor is read and written once, with 128-bit accesses (gfx950
 //     global loads and stores need only 4-byte alignment, so rows of any
-//     width C % 4 == 0 use them; other widths fall back to 32-bit accesses);
+//     width use them, with 32-bit accesses at the ends of rows of odd width;
+//     the embedding forward, the position-embedding gradient, the bias kernels
+//     and rows too wide for the registers move odd widths by 32 bits only);
 //   * a row-wise reduction (layernorm, softmax) gives a row to one wave64 (or,
 //     for the 50k-wide vocabulary rows, one 1024-lane workgroup) that keeps the
 //     whole row in registers between its passes, so the row is fetched once;
@@ -40,11 +42,14 @@ __device__ __forceinline__ float4 ldu4(const float *p) {
     return v;
 }
 __device__ __forceinline__ void stu4(float *p, float4 v) { __builtin_memcpy(p, &v, sizeof(v)); }
-// The same past the caches. For outputs larger than the 256 MB last-level
-// cache, whose lines would only push out what the next kernels read: at 8192 x
-// 50304 (1.65 GB) the cross-entropy backward took 513 us instead of 532 and the
-// softmax 585 instead of 618; at 4096 x 4096 (67 MB) they took 2-3% longer.
-constexpr size_t STREAM_BYTES = 512u << 20;
+// The same past the caches, for outputs that do not fit the 256 MB last-level
+// cache beside the input of the same size and would only push out what the next
+// kernel reads. Softmax and cross-entropy backward one after the other, rows of
+// 50304, streamed and cached, in us: 64 MB of output 56 and 50, 128 MB 100 and
+// 90, 192 MB 148 and 154, 256 MB 194 and 204, 512 MB 365 and 381, 1.6 GB 1112
+// and 1183; the same sign at widths of 300-60000, but for some rows of the
+// softmax (xent_launch).
+constexpr size_t STREAM_BYTES = 160u << 20;
 __device__ __forceinline__ void stu4_nt(float *p, float4 v) {
     typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
     __builtin_nontemporal_store(f4{v.x, v.y, v.z, v.w}, reinterpret_cast<f4 *>(p));
@@ -1076,7 +1081,12 @@ void rows_in_launches(int N, int nt, F &&go) {
 template <int NTHR, int NCH>
 void xent_launch(float *probs, float *losses, const float *logits, const int *targets, int N,
                  int V, int Vp) {
-    const bool stream = (size_t)N * Vp * sizeof(float) >= STREAM_BYTES;
+    // Rows that leave a quarter or more of the 1024 x 8 chunks empty are faster
+    // cached from 1.5 times the cache on (1 GB of 20000 columns 380 us against 406,
+    // of 17000 409 against 453; 28000: 392 against 376; 192 MB of 20000: 86 against 75).
+    const size_t bytes = (size_t)N * Vp * sizeof(float);
+    const bool sparse = NTHR == 1024 && NCH == 8 && V <= 24576 && bytes >= 384u << 20;
+    const bool stream = bytes >= STREAM_BYTES && !sparse;
     auto *kern = Vp % 4 == 0 ? (stream ? softmax_xent_k<NTHR, NCH, false, true>
                                        : softmax_xent_k<NTHR, NCH, false, false>)
                              : (stream ? softmax_xent_k<NTHR, NCH, true, true>

@@ -213,7 +213,9 @@ def test_bias(gpu, N, C):
                                     (5, 65533, 65534), (6, 3, 5), (5, 2, 3),
                                     # the backward's flat map of aligned rows, and both maps of ragged ones
                                     (1000, 127, 128), (33, 1100, 1100), (1000, 65, 65), (301, 257, 257),
-                                    (70, 1537, 1537), (70, 1791, 1791), (70, 1793, 1795)])
+                                    (70, 1537, 1537), (70, 1791, 1791), (70, 1793, 1795),
+                                    # 160 MB and more: stored past the caches
+                                    (840, 50257, 50257), (835, 50257, 50304), (10490, 4000, 4001)])
 def test_softmax_crossentropy(gpu, N, V, Vp):
     r = _rng(6)
     logits = _f32(r.standard_normal((N, Vp)) * 3)
