@@ -622,8 +622,8 @@ def test_k_sliced_tiles(gpu, shape, trans, capfd, monkeypatch):
     bmb.gemm(ta, tb, M, N, K, 0.75, dA.data_ptr(), dB.data_ptr(), 1.25, dC.data_ptr())
     sync("gemm k-sliced")
     err_out = capfd.readouterr().err
-    # Plans are memoised per shape (not per transpose), so the trace line
-    # comes with the first call of a shape, the NN case; the others reuse it.
+    # (A shape that another test has planned already leaves no trace here;
+    # test_k_sliced_plans_and_splits has shapes of its own.)
     plan = [l for l in err_out.splitlines() if "bf16x3 gemm plan %dx%dx%d:" % (M, N, K) in l]
     if trans == (False, False):
         assert plan, err_out
@@ -635,6 +635,38 @@ def test_k_sliced_tiles(gpu, shape, trans, capfd, monkeypatch):
     assert bad == 0 and err < 1e-4, err
     e3, bound = bf16x3_err(got, ta, tb, M, N, K, 0.75, A, B, 1.25, C0)
     assert e3 < bound, (e3, bound)
+
+
+# The 128 x 64 tile in two k-slices (tile 8), and k-sliced tiles whose K is also
+# split into ranges (partials and a reduce), the last range ragged. No other
+# test has these shapes, so every transpose's first call leaves its plan.
+@pytest.mark.parametrize("trans", TRANS, ids=_tag)
+@pytest.mark.parametrize("shape,tiles,split", [((4095, 383, 1151), (8,), False),
+                                               ((3001, 640, 1537), (8, 4, 1), None),
+                                               ((96, 480, 12288), (7,), True),
+                                               ((193, 575, 6143), (4,), True),
+                                               ((66, 1030, 4100), (4, 6), True),
+                                               ((97, 481, 12287), (4,), True)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_k_sliced_plans_and_splits(gpu, shape, tiles, split, trans, capfd, monkeypatch):
+    M, N, K = shape
+    ta, tb = trans
+    A = O.fill_xorshift(M * K, 0x1212)
+    B = O.fill_xorshift(K * N, 0x3434)
+    C0 = O.fill_xorshift(M * N, 0x5656)
+    monkeypatch.setenv("BMB_GEMM_PLAN_TRACE", "1")
+    dA, dB, C = dev(A), dev(B), Guarded(M * N, fill=C0)
+    print("gemm %s %dx%dx%d" % (_tag(trans), M, N, K), flush=True)
+    bmb.gemm(ta, tb, M, N, K, 0.75, dA.data_ptr(), dB.data_ptr(), 1.25, C.ptr)
+    sync("gemm k-sliced")
+    trace = capfd.readouterr().err
+    plan = [l for l in trace.splitlines() if "bf16x3 gemm plan %dx%dx%d:" % (M, N, K) in l]
+    assert plan, trace
+    tile, splits = [int(v) for v in plan[0].split("parts (")[1].split(",")[:2]]
+    assert tile in tiles and split in (None, splits > 1), plan
+    e3, bound = bf16x3_err(C.get(), ta, tb, M, N, K, 0.75, A, B, 1.25, C0)
+    assert e3 < bound, (e3, bound)
+    assert C.ok()
 
 
 # The bf16x3 kernels' edges: rows that end inside a 4-row block, or K inside a

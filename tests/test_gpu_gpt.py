@@ -105,6 +105,36 @@ def test_gradients_at_other_widths(gpu, cfg, b):
         assert bad == 0 and e < 1e-4, (name, e)
 
 
+def test_column_sums_of_a_banded_gelu_gradient(gpu, capfd, monkeypatch):
+    """The FC layer's bias gradient comes from partial sums that the GELU-grad
+    GEMM leaves, one row per wave tile row: here of two bands (256 x 256 tiles,
+    then 64 x 64 with a ragged last one), whose second writes behind the first.
+    Against the column sums of the stored gradient in fp64: chains of fewer
+    than 128 fp32 additions (64 rows of a lane, the lane's other half, up to
+    32 partials of a slice, 32 slices) of at most 2^-24 of the sum of
+    magnitudes each."""
+    cfg, b, t = (1101, 65, 128, 1, 12, 768), 5, 1101
+    n, width = b * t, 4 * 768
+    m = _model(True, cfg=cfg, b=b, t=t)
+    x, y = _batch(77, cfg[1], n)
+    monkeypatch.setenv("BMB_GEMM_PLAN_TRACE", "1")
+    print("gpt banded gelu gradient", cfg, b, flush=True)
+    m.forward(x, y)
+    capfd.readouterr()
+    m.backward()
+    sync("gpt backward")
+    trace = capfd.readouterr().err
+    plans = [l for l in trace.splitlines() if "gemm plan %dx%dx768:" % (n, width) in l]
+    assert plans and "m1 5376" in plans[0] and "parts (0,1,768) (2,1,768)" in plans[0], trace
+    dfch = d2h(m.g.gr.dfch, n * width).reshape(n, width).astype(np.float64)
+    off = _offsets(cfg)
+    i = O.PARAM_NAMES.index("fcb")
+    got = _grads(m)[off[i]:off[i + 1]]
+    bound = 128 * 2.0 ** -24 * np.abs(dfch).sum(axis=0)
+    assert np.all(np.abs(got - dfch.sum(axis=0)) <= bound)
+    assert np.abs(got).max() > 0
+
+
 def _loss_double(m, x, y):
     """Mean loss with the per-position losses summed in fp64 on the host
     (tools/test_grad.cu:44-52)."""
