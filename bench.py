@@ -101,6 +101,9 @@ def parse():
     ap.add_argument("--summarize-trace", metavar="DIR", default=None,
                     help="summarise a rocprofv3 --kernel-trace --marker-trace CSV output "
                          "directory by timed region (no GPU work)")
+    ap.add_argument("--detail", metavar="FILE", default=None,
+                    help="also write every figure (all checks with their errors and bounds) "
+                         "to FILE as JSON")
     ap.add_argument("--region", default=None, help="with --summarize-trace: only this region")
     ap.add_argument("--copy-calib", action="store_true",
                     help="first run a plain 256 MiB device-to-device copy 3 times, the "
@@ -149,6 +152,37 @@ def progress(msg):
     goes to stdout)."""
     print("bench.py [%6.1f s] %s" % (time.perf_counter() - T_START, msg), file=sys.stderr,
           flush=True)
+
+
+def summary_line(line):
+    """The JSON line for stdout: every result of `line`, without what can be
+    computed from them (percentages of a stated ceiling), each check's figures
+    (how many passed, and the one nearest its bound), the clocks of single XCDs
+    and, in the fp32-GEMM step, what the bf16x3 step states already. Under 7,500
+    characters, where the whole is 23,000: a reader that keeps the last few
+    thousand characters of the output still has all of it. --detail writes the
+    whole."""
+    def trim(v):
+        if isinstance(v, dict):
+            return {k: trim(x) for k, x in v.items()
+                    if k not in ("pct_of_own_ceiling", "gfx_clk_mhz_per_xcd", "note")}
+        return v
+
+    out = trim(line)
+    for k, v in line.items():
+        if k.startswith("ladder_"):
+            out[k] = {name: [e["gflops"], e["pct_of_own_peak"]] for name, e in v.items()}
+    fp32 = "config5_gpt_train_step_fp32_gemm"
+    if fp32 in line:
+        out[fp32] = {k: line[fp32][k] for k in ("metric", "value", "unit", "ms_per_step", "steps",
+                                                "warmup", "phase_ms", "loss_first", "loss_last")}
+    v = line["verification"]
+    near = max(v["checks"].items(), key=lambda c: c[1]["err"] / max(c[1]["bound"], 1e-300),
+               default=None)
+    out["verification"] = {"all_ok": v["all_ok"], "failed": v["failed"],
+                           "checks": len(v["checks"]),
+                           "nearest_its_bound": near and dict(near[1], name=near[0])}
+    return json.dumps(out, separators=(",", ":"))
 
 
 def timed(fn, steps, warmup, name="per-launch"):
@@ -743,7 +777,10 @@ def main():
                 cpu = fl
         line["cpu_baseline"] = cpu
     line["verification"] = {"all_ok": not V.failed, "failed": V.failed, "checks": V.checks}
-    print(json.dumps(line))
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(line, f, indent=1)
+    print(summary_line(line))
     if V.failed:
         print("bench.py: verification failed: %s" % ", ".join(V.failed), file=sys.stderr)
         sys.exit(1)
