@@ -45,9 +45,9 @@
 // order is 1-5% faster on the GPT-2 shapes and 2% at N = 4096, bit-identical.
 //
 // What bounds it. With the device full of 128- or 256-wide tiles: power. On
-// N(0, 1) data at N = 4096 the matrix cores are busy 74% of the cycles while
-// the clock falls to 1.7 GHz (2.38 GHz on zeros, 24% faster at the same
-// cycles), so what counts is the energy of everything around the MFMAs.
+// N(0, 1) data at N = 4096 the matrix cores are busy 71% of a launch's cycles
+// while the clock falls to 1.74 GHz; zeros run the same cycles at 2.44 GHz (315
+// and 221 us), so what counts is the energy of everything around the MFMAs.
 // Taking instructions out of the staging (split4 on pairs, loads without
 // address arithmetic, two stages per loop turn) gave 4-5% on 256 x 256 and
 // 6-9% on 128-wide tiles (per 32-k stage and CU: 2.50 -> 2.37 us, 1.42 ->
