@@ -87,8 +87,10 @@ def test_forward_backward_vs_oracle(gpu, use_flash):
 # rows that are no whole tile or wave of rows, a ragged width of the MLP, and a
 # width whose layernorm sums do not fit the fused kernel.
 @pytest.mark.parametrize("cfg,b", [((50, 65, 128, 2, 3, 96), 3), ((33, 65, 66, 1, 1, 32), 1),
-                                   ((8, 65, 128, 1, 16, 2048), 1)],
-                         ids=["C96", "C32", "C2048"])
+                                   ((8, 65, 128, 1, 16, 2048), 1),
+                                   # one and three token rows through every layer
+                                   ((1, 65, 128, 2, 2, 64), 1), ((3, 65, 66, 2, 1, 32), 1)],
+                         ids=["C96", "C32", "C2048", "1row", "3rows"])
 def test_gradients_at_other_widths(gpu, cfg, b):
     n = b * cfg[0]
     m = _model(True, cfg=cfg, b=b, t=cfg[0])
