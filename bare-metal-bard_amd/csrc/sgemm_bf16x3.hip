@@ -609,7 +609,9 @@ struct Bf16x3Gemm {
         // spilled 24-34 of them).
         constexpr int UNROLL = Tl::SMEM_BYTES <= 98304 ? 2 : 1;
         int kt0 = 0;
-        for (const int whole = MODE == SINGLE ? 0 : MODE == SHORT ? (K - 3) / BK : K / BK; kt0 + 1 + UNROLL < whole; kt0 += UNROLL)
+        constexpr int SPARE = MODE == SHORT ? SHORT_K - BK : 0;  // k behind a whole stage
+        const int whole = MODE == SINGLE ? 0 : (K - SPARE) / BK;
+        for (; kt0 + 1 + UNROLL < whole; kt0 += UNROLL)
             static_for<0, UNROLL>([&](auto uc) {
                 const int kt = kt0 + uc, h = UNROLL == 2 ? (int)uc : kt & 1;
                 const __bf16 *st = smem + h * Tl::STAGE;
@@ -1211,10 +1213,10 @@ struct Strides {
 // Whether a tile (in KS k-slices) has a SHORT kernel (short_tile), and for this
 // epilogue: short rows are planned for gemm() only.
 template <class Tl, int KS, int EPI>
-constexpr bool HAS_SHORT = (EPI == bmb::EPI_BLAS || EPI == bmb::EPI_PARTIAL) &&
-                           ((KS == 1 && (std::is_same<Tl, TileM>::value || std::is_same<Tl, TileS>::value)) ||
-                            (KS == 4 && std::is_same<Tl, TileS>::value) ||
-                            (KS == 8 && std::is_same<Tl, TileXS>::value));
+constexpr bool HAS_SHORT =
+    (EPI == bmb::EPI_BLAS || EPI == bmb::EPI_PARTIAL) &&
+    ((KS == 1 && (std::is_same<Tl, TileM>::value || std::is_same<Tl, TileS>::value)) ||
+     (KS == 4 && std::is_same<Tl, TileS>::value) || (KS == 8 && std::is_same<Tl, TileXS>::value));
 
 template <class Tl, bool TA, bool TB, int EPI>
 void launch(int M, int N, int K, const Part &p, float alpha, const float *A, const float *B,

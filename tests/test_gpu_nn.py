@@ -211,7 +211,7 @@ def test_bias(gpu, N, C):
                                     (5, 70000, 70004), (9, 1, 4), (33, 1000, 1000),
                                     (37, 50257, 50257), (9, 1021, 1021), (7, 1022, 1025),
                                     (5, 65533, 65534), (6, 3, 5), (5, 2, 3),
-                                    # the backward's flat map of aligned rows, and both maps of ragged ones
+                                    # the backward's maps: flat (aligned), both (ragged)
                                     (1000, 127, 128), (33, 1100, 1100), (1000, 65, 65), (301, 257, 257),
                                     (70, 1537, 1537), (70, 1791, 1791), (70, 1793, 1795),
                                     # 160 MB and more: stored past the caches
